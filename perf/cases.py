@@ -102,10 +102,11 @@ def draw(rng):
 
 
 class _Maker:
-    """Operands from one seed, on the GPU."""
+    """Operands from one seed, on the GPU; `plain`: each weight as its values in 64 bits instead of laid out."""
 
-    def __init__(self, case, seed):
-        self.pkg = import_package()
+    def __init__(self, case, seed, plain=False):
+        self.plain = plain
+        self.pkg = None if plain else import_package()
         self.dev = torch.device("cuda:0")
         self.gen = torch.Generator(device=self.dev).manual_seed(seed)
         self.fmt, self.group, self.zero = case["fmt"], case.get("group", 0), case.get("zero", False)
@@ -140,6 +141,9 @@ class _Maker:
             scales = (grouped.abs().amax(1) / (half - 0.5)).to(scale_type)
             q = torch.round(grouped / scales.float()[:, None]).clamp(-half, half - 1)
             zeros = None
+        if self.plain:
+            w = q.double() * scales.double()[:, None] + (zeros.double()[:, None] if zeros is not None else 0.0)
+            return (_e4m3(w) if self.fmt == "w4a8" else w).view(k, n), None, None
         q = q.view(k, n).to(torch.int8)
         if not self.group:
             scales = scales.view(n)
@@ -193,10 +197,9 @@ def _pass(state):
     return out
 
 
-def prepare(case, seed):
-    mk = _Maker(case, seed)
+def _operands(mk, case):
     m = case["m"]
-    state = dict(F=mk.pkg.functional, case=case, alpha=0.75)
+    state = dict(case=case, alpha=0.75)
     if case["kind"] == "call":
         state["linear"] = mk.linear(case["k"], case["n"])
         state["x"] = mk.activations(m, case["k"])
@@ -210,8 +213,8 @@ def prepare(case, seed):
         for name, k, n in (("fc1", hidden, 2 * inter), ("fc2", inter, hidden)):
             each = [mk.quantized(k, n) for _ in range(experts)]
             state[name] = dict(k=k, n=n, weight=torch.stack([e[0] for e in each]),
-                               scales=torch.stack([e[1] for e in each]),
-                               zeros=torch.stack([e[2] for e in each]) if case["zero"] else None)
+                               scales=None if mk.plain else torch.stack([e[1] for e in each]),
+                               zeros=torch.stack([e[2] for e in each]) if case["zero"] and not mk.plain else None)
     else:
         hidden, qkv, inter = case["hidden"], case["qkv"], case["inter"]
         sizes = ((hidden, qkv), (hidden, hidden), (hidden, 2 * inter), (inter, hidden))
@@ -222,6 +225,13 @@ def prepare(case, seed):
             state["layers"].append((*linears, norms))
         state["x"], state["x2"] = mk.activations(m, hidden), mk.activations(m, hidden)
         state["attended"], state["gated"] = mk.normal(m, hidden).to(mk.dtype), mk.gated(m, inter)
+    return state
+
+
+def prepare(case, seed):
+    mk = _Maker(case, seed)
+    state = _operands(mk, case)
+    state["F"] = mk.pkg.functional
     if case.get("graph"):
         stream = torch.cuda.Stream()
         stream.wait_stream(torch.cuda.current_stream())
@@ -240,6 +250,49 @@ def run(state):
         state["graph"].replay()
         return state["out"]
     return _pass(state)
+
+
+def _e4m3(x):
+    return x.float().to(torch.float8_e4m3fn).double()
+
+
+def exact(case, seed):
+    """The outputs of `run` in 64 bits.  Where activations and weights become e4m3, that rounding is part of what is
+    asked for and is kept; every other rounding is left out."""
+    mk = _Maker(case, seed, plain=True)
+    st = _operands(mk, case)
+    fp8 = case["fmt"] == "w4a8"
+
+    def linear(lin, x, ready=False):
+        x = x.double()
+        if lin["smooth"] is not None and not ready:
+            x = x * lin["smooth"].double()
+            x = _e4m3(x.to(mk.dtype)) if fp8 else x
+        y = x @ lin["weight"] * (st["alpha"] if fp8 else 1.0)
+        return y if lin["bias"] is None else y + lin["bias"].double()
+
+    def norm(x, gamma, smooth):
+        x = x.double()
+        x = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-5) * gamma.double()
+        return _e4m3((x.to(mk.dtype).double() * smooth.double()).to(mk.dtype))
+
+    if case["kind"] == "call":
+        return [linear(st["linear"], st["x"])]
+    if case["kind"] == "experts":
+        ends = st["rows_before"].tolist()
+        pick = [slice(begin, end) for begin, end in zip([0] + ends[:-1], ends)]
+        x = st["x"].double()
+        both = torch.cat([x[rows] @ w for rows, w in zip(pick, st["fc1"]["weight"])])
+        value, gate = both.chunk(2, dim=1)
+        hidden = value * torch.nn.functional.silu(gate)
+        return [hidden, torch.cat([hidden[rows] @ w for rows, w in zip(pick, st["fc2"]["weight"])])]
+    out = []
+    for qkv, o_proj, gate_up, down, norms in st["layers"]:
+        x, x2 = st["x"], st["x2"]
+        if fp8:
+            x, x2 = norm(x, norms[0], qkv["smooth"]), norm(x2, norms[1], gate_up["smooth"])
+        out += [linear(qkv, x, fp8), linear(o_proj, st["attended"]), linear(gate_up, x2, fp8), linear(down, st["gated"])]
+    return out
 
 
 def _matmul_work(case, m, k, n, n_out=None, matrices=1.0):
