@@ -31,7 +31,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-command-line-argum
           "-ffp-contract=off"]
 # Per-file additions.  The skinny-M kernel reads its MFMA results with VALU instructions every
 # group: keep those accumulators in the architectural VGPRs instead of copying them out of AGPRs.
-PER_FILE = {"skinny_": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+PER_FILE = {"skinny_": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "mid_": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def sources():

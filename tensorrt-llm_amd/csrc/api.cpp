@@ -30,6 +30,10 @@ int launch_skinny_BF16_4(MatmulProblem const& p, GemmPlan const& plan, void* str
 int launch_skinny_BF16_8(MatmulProblem const& p, GemmPlan const& plan, void* stream);
 int launch_skinny_FP16_4(MatmulProblem const& p, GemmPlan const& plan, void* stream);
 int launch_skinny_FP16_8(MatmulProblem const& p, GemmPlan const& plan, void* stream);
+int launch_mid_BF16_4(MatmulProblem const& p, MidPlan const& plan, void* stream);
+int launch_mid_BF16_8(MatmulProblem const& p, MidPlan const& plan, void* stream);
+int launch_mid_FP16_4(MatmulProblem const& p, MidPlan const& plan, void* stream);
+int launch_mid_FP16_8(MatmulProblem const& p, MidPlan const& plan, void* stream);
 int launch_gemm_w4a8(MatmulProblem const& p, void* stream);
 int launch_stream_w4a8(MatmulProblem const& p, void* stream);
 
@@ -52,11 +56,47 @@ GemmPlan planned_gemm(int m, int n, int k, int bits, int group)
     return plan_gemm(m, n, k, bits, true, 1, group);
 }
 
+// The barrier-free mid-M kernel (mid_kernel.h) for this problem, and its launch shape: where mid_cost_us estimates it
+// cheaper than `other_us`, the estimate of the kernel the regime would run.  Measured against those (bf16, group 128,
+// zeros; us, old -> new): 4096 x 4096 at 32 / 48 / 64 / 96 / 160 rows 10.5 -> 7.9 / 14.2 -> 9.6 / 15.7 -> 10.2 / 18.7 ->
+// 10.6 / 20.8 -> 13.6; 4096 x 6144 at 48 rows 16.0 -> 10.7; 14336 x 4096 19.2 -> 17.6; 4096 x 28672 at 32 / 48 rows
+// 20.5 -> 20.2 / 27.5 -> 23.7, at 64 rows slower (30 -> 36): the wide matrices keep the tiled kernels from there on.
+// WOQ_MID_SHAPE="rt,ns,waves,splits" forces it where it can run, "0" switches it off.
+bool pick_mid_shape(MatmulProblem const& p, double other_us, MidPlan& plan)
+{
+    EnvOverrides const& env = env_overrides();
+    if (env.mid_mode == 0 || p.w4a8 || p.pre_quant_scale || p.num_experts || p.activation != WOQ_ACT_IDENTITY || p.residual
+        || p.k % tile_k_of_bits(p.bits) || (p.group_size != 0 && (p.bits == 8 || p.group_size > 128)))
+        return false;
+    if (env.mid_mode == 1)
+    {
+        plan = MidPlan{env.mid_shape[0], env.mid_shape[1], env.mid_shape[2], env.mid_shape[3]};
+        return true;
+    }
+    if (!p.built_in_choice || p.m <= 16 || p.m > kMidMaxM)
+        return false;
+    double const t = best_mid_plan(p.m, p.n, p.k, p.bits, p.group_size, p.workspace ? p.workspace_bytes : 0, plan);
+    // (0.88: with the two models' errors, 3 of 95 measured problems end up slower than before, by 1 ... 7 %, and the choice
+    // costs 2 % on average against the better of the two; at 1.0 a few lose 10 % and the average gains nothing)
+    return t > 0 && t < 0.88 * other_us;
+}
+
+int launch_mid(MatmulProblem const& p, MidPlan const& plan, void* stream)
+{
+    if (p.out_dtype == WOQ_BF16)
+        return p.bits == 4 ? launch_mid_BF16_4(p, plan, stream) : launch_mid_BF16_8(p, plan, stream);
+    return p.bits == 4 ? launch_mid_FP16_4(p, plan, stream) : launch_mid_FP16_8(p, plan, stream);
+}
+
 int launch_gemm(MatmulProblem const& p, void* stream)
 {
     if (p.w4a8)
         return launch_gemm_w4a8(p, stream);
-    return launch_gemm_planned(p, planned_gemm(p.m, p.n, p.k, p.bits, p.group_size), stream);
+    GemmPlan const plan = planned_gemm(p.m, p.n, p.k, p.bits, p.group_size);
+    MidPlan mid;
+    if (pick_mid_shape(p, plan.cost_us, mid))
+        return launch_mid(p, mid, stream);
+    return launch_gemm_planned(p, plan, stream);
 }
 
 int launch_gemm_planned(MatmulProblem const& p, GemmPlan const& plan, void* stream)
@@ -80,6 +120,9 @@ int launch_stream(MatmulProblem const& p, void* stream)
     if (!p.num_experts && p.m > kStreamMaxM) // a grouped problem runs 16-row passes per expert
         return fail(WOQ_ERR_UNSUPPORTED, "unsupported m: the streaming kernel covers m <= %d (got %d)", kStreamMaxM,
             p.m);
+    MidPlan mid;
+    if (pick_mid_shape(p, p.m > 16 ? stream_cost_us(p.m, p.n, p.k) : 0.0, mid))
+        return launch_mid(p, mid, stream);
     if (p.out_dtype == WOQ_BF16)
         return p.bits == 4 ? launch_stream_BF16_4(p, stream) : launch_stream_BF16_8(p, stream);
     return p.bits == 4 ? launch_stream_FP16_4(p, stream) : launch_stream_FP16_8(p, stream);
@@ -559,6 +602,8 @@ EnvOverrides read_env()
         o.stream_splits = std::atoi(e);
     if (char const* e = std::getenv("WOQ_GEMM_PERSIST"))
         o.persist_off = e[0] == '0';
+    if (char const* e = std::getenv("WOQ_MID_SHAPE"))
+        o.mid_mode = std::sscanf(e, "%d,%d,%d,%d", &o.mid_shape[0], &o.mid_shape[1], &o.mid_shape[2], &o.mid_shape[3]) == 4 ? 1 : 0;
     return o;
 }
 
@@ -870,6 +915,9 @@ static int run_matmul(const woq_matmul_args* args, void* stream)
     validate(args, p);
     if (p.m == 0)
         return WOQ_OK;
+    EnvOverrides const& env = env_overrides();
+    p.built_in_choice = args->regime == WOQ_REGIME_AUTO && env.regime == WOQ_REGIME_AUTO && !current_tactic()
+        && !env.gemm_kernel && !env.gemm_rt && !env.gemm_splits && !env.has_stream_shape && !env.stream_splits;
     bool const streaming = pick_regime(args) == WOQ_REGIME_STREAM;
     if (streaming && !p.w4a8)
         return launch_stream(p, stream); // smoothing is fused into the 16-bit streaming kernel

@@ -31,6 +31,7 @@ inline int bits_of(int quant_type)
 //   WOQ_STREAM_SLOTS=0                WOQ_GEMM_KERNEL=exact|skinny       WOQ_GEMM_RT=4|8|16
 //   WOQ_GEMM_SPLITS=<n>               WOQ_STREAM_SPLITS=<n>              WOQ_GEMM_PERSIST=0
 //   WOQ_GEMM_COLS=192|256             WOQ_ROW_SHAPE=waves,tiles | 0      WOQ_ROWS_SHAPE=waves,ns,tiles | 0
+//   WOQ_MID_SHAPE=rt,ns,waves,splits | 0
 struct EnvOverrides
 {
     int regime = 0;                // woq_regime; 0 = none
@@ -49,6 +50,8 @@ struct EnvOverrides
     int gemm_splits = 0;           // K split of the GEMM regime
     int stream_splits = 0;         // K slices of the streaming kernel (0 = built-in rule)
     bool persist_off = false;      // WOQ_GEMM_PERSIST=0: no persistent prefill kernels
+    int mid_mode = -1;             // barrier-free mid-M kernel (mid_kernel.h): -1 built-in rule, 0 off, 1 forced shape
+    int mid_shape[4] = {0, 0, 0, 0}; // row tiles and strips per workgroup, wavefronts, K split
 };
 EnvOverrides const& env_overrides();
 
@@ -86,6 +89,7 @@ struct MatmulProblem
     size_t weight_stride = 0, scale_stride = 0;
     int activation = 5;             // WOQ_ACT_IDENTITY; see woq_grouped_matmul
     void const* residual = nullptr; // [m, n_out] in the output type, added after the activation
+    bool built_in_choice = false;   // neither the caller nor the environment nor a tactic fixed the regime or kernel
 };
 
 // kernel launchers (each returns a woq_status)
@@ -109,6 +113,12 @@ struct GemmPlan
     int k_splits;
     size_t ws_bytes;
     double cost_us; // the cost model's estimate (plan_gemm only)
+};
+
+// How the barrier-free mid-M kernel runs a problem: row tiles and strips per workgroup, wavefronts, K split.
+struct MidPlan
+{
+    int rt, ns, waves, splits;
 };
 
 // float32 partial sums of a K split: one [m, n] slab per slice of K
@@ -298,6 +308,72 @@ inline GemmPlan plan_gemm_w4a8(int m, int n, int k)
     return pl;
 }
 
+// Estimated time (microseconds) of the barrier-free mid-M kernel (mid_kernel.h) at one launch shape, fitted to 113
+// problems x up to ten shapes (K = 2048 ... 14336, N = 2048 ... 28672, 24 ... 160 rows; int4 group 128 / 64 / per-channel,
+// int8 per-channel): mean error 5-7 %, and picking the shape by it costs 1-2 % on average against the best one.
+//   * a wavefront spends a + b * rt * ns + c * ns + e * rt microseconds per tile row of K with its SIMD shared by two
+//     wavefronts, `half` of it where four-wavefront workgroups leave every CU with a single one;
+//   * eight-wavefront workgroups run one per CU, four-wavefront ones two per CU;
+//   * prologue and reduction cost `pro` + `red` * rt * ns per round; a launch cannot beat its weights' read at `read`
+//     bytes per picosecond; a K split adds a launch and the float32 slabs.
+inline double mid_cost_us(MidPlan const& pl, int m, int n, int k, int bits, int group)
+{
+    struct Fit
+    {
+        double t0, pro, a, b, c, e, half, read, split, red;
+    };
+    static constexpr Fit kInt4G128{2.016, 1.274, 0.470, 0.0995, 0.0, 0.167, 0.594, 3.46, 1.98, 0.199};
+    static constexpr Fit kInt4G64{2.367, 0.476, 0.472, 0.169, 0.0, 0.145, 0.607, 4.09, 2.43, 0.222};
+    static constexpr Fit kInt4Channel{2.576, 0.235, 0.316, 0.0, 0.148, 0.307, 0.534, 5.36, 2.49, 0.176};
+    static constexpr Fit kInt8Channel{2.744, 0.278, 0.200, 0.0, 0.139, 0.178, 0.517, 6.59, 2.69, 0.153};
+    Fit const& f = bits == 8 ? kInt8Channel : (group == 0 ? kInt4Channel : (group == 64 ? kInt4G64 : kInt4G128));
+    int const k_tiles = k / tile_k_of_bits(bits), strips = n / kTileN;
+    long const groups = ((strips + pl.ns - 1) / pl.ns + 7) / 8 * 8;
+    long const wgs = groups * ((m + pl.rt * 16 - 1) / (pl.rt * 16)) * pl.splits;
+    int const iters = ((k_tiles + pl.splits - 1) / pl.splits + pl.waves - 1) / pl.waves;
+    double const work = iters * (f.a + f.b * pl.rt * pl.ns + f.c * pl.ns + f.e * pl.rt);
+    double const fixed = f.pro + f.red * pl.rt * pl.ns;
+    double t;
+    if (pl.waves == 8)
+        t = (double) ((wgs + 255) / 256) * (work + fixed);
+    else
+    {
+        long const left = wgs % 512;
+        t = (double) (wgs / 512) * (work + fixed) + (left > 256 ? work + fixed : (left > 0 ? f.half * work + fixed : 0.0));
+    }
+    double const bytes = (double) k * n * bits / 8;
+    t = f.t0 + (t > bytes / (f.read * 1e6) ? t : bytes / (f.read * 1e6));
+    if (pl.splits > 1)
+        t += f.split + (double) m * n * 4.0 * pl.splits * 3.3e-7;
+    return t;
+}
+
+// The launch shape mid_cost_us estimates cheapest with at most `ws_bytes` of float32 slabs, and its cost.  17 rows and
+// more: one row tile per 16 of them up to four, several workgroups of three or four row tiles beyond.
+inline double best_mid_plan(int m, int n, int k, int bits, int group, size_t ws_bytes, MidPlan& best)
+{
+    static constexpr int kShapes[][2] = {{1, 8}, {2, 8}, {4, 4}, {4, 8}}; // strips, wavefronts
+    int const k_tiles = k / tile_k_of_bits(bits);
+    int const row_tiles = (m + 15) / 16;
+    double cost = 0;
+    bool have = false;
+    for (int rt = row_tiles <= 4 ? row_tiles : 3; rt <= (row_tiles <= 4 ? row_tiles : 4); ++rt)
+        for (auto const& sh : kShapes)
+            for (int splits = 1; splits <= 4; splits *= 2)
+            {
+                // (rt, ns) pairs whose sums, with group scales twice, do not fit the register file are not built
+                if (rt < 2 || (group != 0 && sh[0] == 4 && rt >= (group == 64 ? 3 : 4)))
+                    continue;
+                if (k_tiles / splits < sh[1] || (splits > 1 && split_partial_bytes(m, n, splits) > ws_bytes))
+                    continue;
+                MidPlan const pl{rt, sh[0], sh[1], splits};
+                double const t = mid_cost_us(pl, m, n, k, bits, group);
+                if (!have || t < cost)
+                    have = true, cost = t, best = pl;
+            }
+    return have ? cost : -1.0;
+}
+
 // One way to run a 16-bit problem: the regime and, inside it, the streaming kernel's launch shape
 // (for problems of `mt` 16-row tiles) or the GEMM kernel, tile height and K split.  Counterpart of
 // the reference's CutlassGemmConfig with its enableCudaKernel pseudo-tactic
@@ -333,6 +409,7 @@ int raise_lds_once(std::atomic<uint64_t>& raised, void const* kernel, int bytes)
 constexpr int kStreamMaxM = 128;
 constexpr int kStreamW4a8MaxM = 32;     // rows the W4A8 streaming kernel covers (two 16-row tiles per wavefront above 16)
 constexpr int kStreamW4a8AutoMaxM = 16; // rows up to which the built-in rule takes it
+constexpr int kMidMaxM = 160;           // rows up to which the barrier-free mid-M kernel is considered
 // most LDS a streaming workgroup stages its operands in (activations, group scales and zeros, row
 // sums): what the CU's 160 KiB leave next to the static reduction buffer of the epilogue
 // (`slots` = strips per wavefront x 16-row tiles, 256 floats per slot and wavefront)

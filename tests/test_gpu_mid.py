@@ -1,0 +1,104 @@
+"""The barrier-free mid-M kernel (csrc/kernels/mid_kernel.h): every instantiated launch shape against the float64
+oracle at the edges of its tiles, the same call on the general kernels, and the rule that picks it."""
+import numpy as np
+import pytest
+import torch
+
+from _util import parity_err, random_problem, run_product
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-2  # the repository's bar: the 16-bit output rounding and the weights' own
+SHAPES = [(1, 8), (2, 8), (4, 4), (4, 8)]
+
+
+def _last_launch(pkg):
+    return (pkg._lib.lib.woq_last_launch() or b"").decode()
+
+
+def _instantiated(rt, ns, group):
+    return group == 0 or ns < 4 or rt < (3 if group == 64 else 4)
+
+
+@pytest.mark.parametrize("rt", [2, 3, 4])
+@pytest.mark.parametrize("bits,group,dtype", [(4, 128, "bf16"), (4, 64, "fp16"), (4, 0, "bf16"), (8, 0, "fp16"),
+                                              (8, 0, "bf16"), (4, 128, "fp16"), (4, 64, "bf16")])
+def test_mid_every_shape(pkg, oracle, dev, woq_env, rt, bits, group, dtype):
+    """Strips that do not divide by a workgroup's, one row past a row tile / a whole tile / a second tile of rows, tile
+    rows of K that leave some wavefronts one more than others (or none), K split with a last slice that is shorter;
+    zeros, bias and smoothing on and off; the same bits on every call."""
+    tk = 128 if bits == 4 else 64
+    for ns, waves in SHAPES:
+        if not _instantiated(rt, ns, group):
+            continue
+        for M, tiles, N, splits in [(16 * rt - 15, 9, 16 * 9, 1), (16 * rt, 21, 16 * 11, 2), (16 * rt + 1, 13, 16 * 8, 1),
+                                    (32 * rt + 7, 37, 16 * 3, 4)]:
+            woq_env(WOQ_MID_SHAPE="%d,%d,%d,%d" % (rt, ns, waves, splits))
+            full = splits == 2
+            p = random_problem(oracle, M, tk * tiles, N, bits, group, dtype, zero=group != 0 and M % 2 == 1, bias=full,
+                               pqs=full, seed=M + tiles + ns)
+            out = run_product(pkg, oracle, dev, p, 2)  # (the tiled regime smooths in a pass of its own)
+            assert "mid rt=%d ns=%d waves=%d splits=%d" % (rt, ns, waves, splits) in _last_launch(pkg), _last_launch(pkg)
+            assert parity_err(oracle, out, p) < TOL, (ns, waves, M, tiles, N, splits)
+            again = run_product(pkg, oracle, dev, p, 2)
+            assert (again.view(np.uint32) == out.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("bits,group", [(4, 128), (4, 64), (4, 0), (8, 0)])
+def test_mid_against_the_general_path(pkg, oracle, dev, woq_env, bits, group):
+    """One-hot activations return single weights times their scale, on this kernel and on the one it replaces; infinities
+    and NaN in one row stay in that row."""
+    K, N, M = 2048, 1040, 40
+    p = random_problem(oracle, M, K, N, bits, group, "bf16", zero=group != 0, seed=group + bits)
+    p["act"] = np.zeros((M, K), np.float32)
+    for r in range(M):
+        p["act"][r, (53 * r + 7) % K] = 1.0
+    p["act"][3, 100] = np.inf
+    p["act"][5, 200] = np.nan
+    outs = []
+    for shape in (None, "0"):
+        woq_env(WOQ_MID_SHAPE=shape)
+        outs.append(run_product(pkg, oracle, dev, p, 0))
+        assert ("mid" in _last_launch(pkg)) == (shape is None), _last_launch(pkg)
+    w = oracle.dequantize(p["q"], p["scales"], p["zeros"], group, "bf16")
+    for out in outs:
+        for r in range(M):
+            if r in (3, 5):
+                assert not np.isfinite(out[r]).any()
+                continue
+            row = w[(53 * r + 7) % K]
+            # one output rounding (2^-8) on top of the weight's own in `w`
+            assert (np.abs(out[r] - row) <= np.abs(row) * 2.0 ** -7 + 2.5e-7).all(), r
+
+
+def test_mid_rule(pkg, oracle, dev, woq_env):
+    """Taken on narrow matrices from 17 rows on when nothing is forced; not for one row tile, wide matrices at 64 rows,
+    flexible groups, int8 with group scales, a K that is no multiple of the weight tile, or a regime the caller named."""
+    woq_env(WOQ_MID_SHAPE=None)
+    run = lambda M, K, N, bits, group, regime=0: (run_product(
+        pkg, oracle, dev, random_problem(oracle, M, K, N, bits, group, "bf16", seed=M), regime), _last_launch(pkg))[1]
+    for M in (17, 33, 48, 64, 65, 160):
+        assert "mid" in run(M, 4096, 1024, 4, 128), M
+    assert "mid" in run(48, 4096, 1024, 8, 0)
+    for args in [(16, 4096, 1024, 4, 128), (161, 4096, 1024, 4, 128), (48, 4096, 1024, 4, 256), (48, 4096, 1024, 8, 128),
+                 (48, 2112, 1024, 4, 64)]:
+        assert "mid" not in run(*args), args
+    for regime in (1, 2):
+        assert "mid" not in run(48, 4096, 1024, 4, 128, regime)
+
+
+def test_mid_split_only_with_room(pkg, oracle, dev, woq_env):
+    """A long K on few columns splits K when the workspace holds the slabs and runs without a split otherwise."""
+    F = pkg.functional
+    from _util import preprocess, to_dev
+    M, K, N = 48, 7168, 512
+    p = random_problem(oracle, M, K, N, 4, 128, "bf16", zero=True, bias=True, seed=5)
+    woq_env(WOQ_MID_SHAPE=None)
+    w = preprocess(pkg, oracle, p["q"], 4).to(dev)
+    need = pkg._lib.lib.woq_workspace_bytes(M, N, K, F.ZERO | F.BIAS, pkg._lib.BF16)
+    for ws in (torch.full((need,), 0x7F, dtype=torch.uint8, device=dev), torch.full((64 << 20,), 0x7F, dtype=torch.uint8, device=dev)):
+        for _ in range(2):
+            out = F.woq_matmul_raw(to_dev(p["act"], "bf16", dev), None, w, to_dev(p["scales"], "bf16", dev),
+                                   to_dev(p["zeros"], "bf16", dev), to_dev(p["bias"], "bf16", dev), n=N, k=K, group_size=128,
+                                   quant_algo=F.ZERO | F.BIAS, workspace=ws)
+            torch.cuda.synchronize()
+            assert parity_err(oracle, out.float().cpu().numpy(), p) < TOL
