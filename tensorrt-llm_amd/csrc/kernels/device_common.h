@@ -208,6 +208,38 @@ __device__ __forceinline__ u32x4 expand_int4(uint32_t w, NibbleConsts const& c)
     return r;
 }
 
+// The same with a small base, for kernels whose sums run over a long K before BASE times the row sum is taken out again:
+// out = s * (P - OFFSET * S) loses OFFSET / |q| of the float32 sums' precision, a factor of 200 with fp16's 1024 + u
+// (per-channel scales, K = 14336: error against 64 bits 5.4e-4 where an exact conversion has 2.1e-4).  fp16 holds 16 + u
+// with the nibble at bits 6 ... 9 (ulp 1/64), for one shift more per operand; bf16's 128 + u is far below its own output
+// rounding and stays.
+template <int DT>
+struct Fine4
+{
+    static constexpr float kOffset = DT == WOQ_FP16 ? 16.f + 8.f : Elem<DT>::kBase4 + 8.f;
+};
+
+template <int DT>
+__device__ __forceinline__ NibbleConsts fine_nibble_consts()
+{
+    NibbleConsts c;
+    c.mask = DT == WOQ_FP16 ? 0x03C003C0u : 0x000F000Fu;
+    c.magic = DT == WOQ_FP16 ? 0x4C004C00u : Elem<DT>::kMagic4;
+    asm volatile("" : "+s"(c.mask));
+    asm volatile("" : "+v"(c.magic));
+    return c;
+}
+
+// operand register `pr` (elements 2 pr, 2 pr + 1)
+template <int DT>
+__device__ __forceinline__ uint32_t expand_int4_fine_reg(uint32_t w, int pr, NibbleConsts const& c)
+{
+    if constexpr (DT == WOQ_FP16)
+        return ((pr < 2 ? w << (6 - 4 * pr) : w >> (4 * pr - 6)) & c.mask) | c.magic;
+    else
+        return ((w >> (4 * pr)) & c.mask) | c.magic;
+}
+
 // int8: two dwords hold elements 0..3 and 4..7 as bytes.
 template <int DT>
 __device__ __forceinline__ u32x4 expand_int8(uint32_t w0, uint32_t w1);

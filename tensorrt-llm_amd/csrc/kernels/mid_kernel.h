@@ -57,7 +57,7 @@ mid_kernel(void const* weight, void const* act, void const* scales, void const* 
     constexpr bool PER_CHANNEL = GROUP == 0;
     constexpr int SEGS = (!PER_CHANNEL && GROUP < TK) ? TK / GROUP : 1; // scale groups inside a tile row
     constexpr int SEG_SLABS = SLABS / SEGS;
-    constexpr float OFF = Offset<DT, BITS>::value;
+    constexpr float OFF = BITS == 4 ? Fine4<DT>::kOffset : Offset<DT, BITS>::value;
     constexpr uint32_t kOob = 0x80000000u;
     constexpr int UNITS = SLABS / 2;            // units of 64 rows of K in a tile row
     constexpr int UNIT_BYTES = 2 * RT * 1024;   // activation fragments of one unit
@@ -172,12 +172,13 @@ mid_kernel(void const* weight, void const* act, void const* scales, void const* 
     };
 
     u32x4 const ones = {E::kOnes, E::kOnes, E::kOnes, E::kOnes};
-    NibbleConsts const nib = nibble_consts<DT>();
+    NibbleConsts const nib = fine_nibble_consts<DT>();
     f32x4 const zero4 = {0.f, 0.f, 0.f, 0.f};
     auto expand = [&](u32x4 const& wv, int j) -> u32x4
     {
         if constexpr (BITS == 4)
-            return expand_int4<DT>(wv[j], nib);
+            return u32x4{expand_int4_fine_reg<DT>(wv[j], 0, nib), expand_int4_fine_reg<DT>(wv[j], 1, nib),
+                expand_int4_fine_reg<DT>(wv[j], 2, nib), expand_int4_fine_reg<DT>(wv[j], 3, nib)};
         else
             return expand_int8<DT>(wv[2 * j], wv[2 * j + 1]);
     };

@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves
     constexpr int SEGS = TK / SEG;
     constexpr int SEG_SLABS = SEG / 32;
     constexpr int A_BYTES = kSkinnyBM * TK * 2;
-    constexpr float OFF = Offset<DT, BITS>::value;
+    constexpr float OFF = BITS == 4 ? Fine4<DT>::kOffset : Offset<DT, BITS>::value;
 
     constexpr int SC_SLOTS = GROUP != 0 ? SEGS * (ZERO ? 2 : 1) : 0; // 256-byte scale slots per wavefront and step
 
@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves
 
     f32x4 const zero4 = {0.f, 0.f, 0.f, 0.f};
     u32x4 const ones = {E::kOnes, E::kOnes, E::kOnes, E::kOnes};
-    [[maybe_unused]] NibbleConsts const nib = nibble_consts<DT>();
+    [[maybe_unused]] NibbleConsts const nib = fine_nibble_consts<DT>();
 
     // acc: finished sums (GROUP != 0) or the running P (per-channel scales are applied at the end);
     // acc_s: the running S of the per-channel mode
@@ -229,7 +229,7 @@ __global__ void __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves
     auto expand_reg = [&](u32x4 const& w, int j, int pr) -> uint32_t
     {
         if constexpr (BITS == 4)
-            return ((w[j] >> (4 * pr)) & nib.mask) | nib.magic;
+            return expand_int4_fine_reg<DT>(w[j], pr, nib);
         else
             return expand_int8_reg<DT>(w[2 * j + pr / 2], pr % 2);
     };
