@@ -40,7 +40,8 @@ int launch_stream_w4a8(MatmulProblem const& p, void* stream);
 int launch_gemm_planned(MatmulProblem const& p, GemmPlan const& plan, void* stream);
 
 // plan of a plain (not grouped) 16-bit GEMM-regime call: the tactic in force, else the cost model's
-GemmPlan planned_gemm(int m, int n, int k, int bits, int group)
+// (`ws_limit`, `contract`: see plan_gemm)
+GemmPlan planned_gemm(int m, int n, int k, int bits, int group, size_t ws_limit = (size_t) -1, bool contract = false)
 {
     Tactic const* t = current_tactic();
     if (t && t->regime == WOQ_REGIME_GEMM && t->rt != 0 && (t->rt != 2 || (t->skinny && bits == 4)))
@@ -53,7 +54,7 @@ GemmPlan planned_gemm(int m, int n, int k, int bits, int group)
         pl.ws_bytes = split_partial_bytes(m, n, pl.k_splits);
         return pl;
     }
-    return plan_gemm(m, n, k, bits, true, 1, group);
+    return plan_gemm(m, n, k, bits, true, 1, group, ws_limit, contract);
 }
 
 // The barrier-free mid-M kernel (mid_kernel.h) for this problem, and its launch shape: where mid_cost_us estimates it
@@ -92,7 +93,7 @@ int launch_gemm(MatmulProblem const& p, void* stream)
 {
     if (p.w4a8)
         return launch_gemm_w4a8(p, stream);
-    GemmPlan const plan = planned_gemm(p.m, p.n, p.k, p.bits, p.group_size);
+    GemmPlan const plan = planned_gemm(p.m, p.n, p.k, p.bits, p.group_size, p.workspace ? p.workspace_bytes : 0);
     MidPlan mid;
     if (pick_mid_shape(p, plan.cost_us, mid))
         return launch_mid(p, mid, stream);
@@ -594,7 +595,7 @@ EnvOverrides read_env()
     if (char const* e = std::getenv("WOQ_GEMM_RT"))
     {
         int const v = std::atoi(e);
-        o.gemm_rt = (v == 4 || v == 8 || v == 16) ? v : 0;
+        o.gemm_rt = (v == 4 || v == 8 || v == 10 || v == 12 || v == 16) ? v : 0;
     }
     if (char const* e = std::getenv("WOQ_GEMM_SPLITS"))
         o.gemm_splits = std::atoi(e);
@@ -773,7 +774,7 @@ extern "C" int woq_select_regime(int32_t m, int32_t n, int32_t k, int32_t quant_
     if (m <= 64)
     {
         int const bits = (quant_algo & WOQ_ALGO_INT8_WEIGHT) ? 8 : 4;
-        if (stream_cost_us(m, n, k) < plan_gemm(m, n, k, bits).cost_us)
+        if (stream_cost_us(m, n, k) < plan_gemm(m, n, k, bits, true, 1, -1, (size_t) -1, true).cost_us)
             return WOQ_REGIME_STREAM;
     }
     return WOQ_REGIME_GEMM;
@@ -810,17 +811,25 @@ static size_t stream_workspace_bytes(int m, int n, int k, int quant_algo)
 }
 
 // float32 partial buffer of one GEMM-regime call with exactly m rows
-// (group: the problem's group size, or -1 for a caller that does not know it - the plan may depend on
-// it, so such a caller gets the larger of the candidates)
+// (group: the problem's group size - then what the call has to bring - or -1: what the best plan of any group size
+// could use)
 static size_t split_bytes(int m, int n, int k, int quant_algo, int group = -1)
 {
     if (quant_algo & WOQ_ALGO_FP8_ALPHA)
         return plan_gemm_w4a8(m, n, k).ws_bytes;
     int const bits = (quant_algo & WOQ_ALGO_INT8_WEIGHT) ? 8 : 4;
     if (group >= 0)
-        return planned_gemm(m, n, k, bits, group).ws_bytes;
-    size_t const a = planned_gemm(m, n, k, bits, -1).ws_bytes, b = planned_gemm(m, n, k, bits, 128).ws_bytes;
-    return a > b ? a : b;
+        return planned_gemm(m, n, k, bits, group, (size_t) -1, true).ws_bytes;
+    size_t bytes = 0;
+    for (int g : {-1, 0, 128}) // the estimates differ between these classes
+        for (bool contract : {false, true}) // (an old estimate knows no per-channel class)
+        {
+            if (contract && g == 0)
+                continue;
+            size_t const b = planned_gemm(m, n, k, bits, g, (size_t) -1, contract).ws_bytes;
+            bytes = b > bytes ? b : bytes;
+        }
+    return bytes;
 }
 
 // what one GEMM-regime call with exactly m rows uses
@@ -829,16 +838,24 @@ static size_t gemm_workspace_bytes(int m, int n, int k, int quant_algo, int grou
     return smooth_bytes(m, k, quant_algo) + split_bytes(m, n, k, quant_algo, group);
 }
 
-extern "C" size_t woq_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t quant_algo, int32_t act_dtype)
+// The most split_bytes of any row count up to m, remembered per thread for the last problems asked about: a pure
+// function of its arguments and the environment overrides (a set of which is never changed once in force), and a host
+// program asks for it in front of every call (8192 rows, 14336 x 4096: 190 us to compute, 40 before there were six
+// estimates to take the largest of).
+static size_t largest_split_bytes(int m, int n, int k, int quant_algo)
 {
-    (void) act_dtype;
-    if (m <= 0 || k <= 0 || n <= 0)
-        return 0;
-    // Enough for every call with at most m rows (the reference sizes its workspace for the
-    // profile's largest M the same way), in either regime.  The smoothing region grows with m;
-    // the split-K region does not (large m does not split, small m splits most), so take its
-    // maximum over the row counts up to m.
-    size_t bytes = smooth_bytes(m, k, quant_algo);
+    struct Known
+    {
+        EnvOverrides const* env;
+        int m, n, k, quant_algo;
+        size_t bytes;
+    };
+    static thread_local Known known[64];
+    EnvOverrides const* const env = &env_overrides();
+    uint32_t const hash = (uint32_t) m * 2654435761u ^ (uint32_t) n * 2246822519u ^ (uint32_t) k * 3266489917u ^ (uint32_t) quant_algo;
+    Known& e = known[(hash >> 16) % 64];
+    if (e.env == env && e.m == m && e.n == n && e.k == k && e.quant_algo == quant_algo && !current_tactic())
+        return e.bytes;
     // A plan splits K only while tiles * splits <= 512, which even the tallest (256-row) tiles exceed
     // beyond 256 * (256 / column tiles) rows; below that the plan may change at any row count.
     // Within a class of 16 rows every candidate has the same tiles, and the partial traffic, which
@@ -854,6 +871,22 @@ extern "C" size_t woq_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t q
         size_t const per_row = split_bytes(lo, n, k, quant_algo) / (size_t) lo;
         split = per_row * hi > split ? per_row * hi : split;
     }
+    if (!current_tactic())
+        e = Known{env, m, n, k, quant_algo, split};
+    return split;
+}
+
+extern "C" size_t woq_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t quant_algo, int32_t act_dtype)
+{
+    (void) act_dtype;
+    if (m <= 0 || k <= 0 || n <= 0)
+        return 0;
+    // Enough for every call with at most m rows (the reference sizes its workspace for the
+    // profile's largest M the same way), in either regime.  The smoothing region grows with m;
+    // the split-K region does not (large m does not split, small m splits most), so take its
+    // maximum over the row counts up to m.
+    size_t bytes = smooth_bytes(m, k, quant_algo);
+    size_t const split = largest_split_bytes(m, n, k, quant_algo);
     size_t const tuned = tuned_split_bytes(m, n, k, quant_algo);
     bytes += split > tuned ? split : tuned;
     // the streaming regime's own K split (16-bit activations, at most 16 rows)

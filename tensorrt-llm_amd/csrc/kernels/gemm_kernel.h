@@ -30,12 +30,16 @@ namespace woq
 
 constexpr int kGemmGroupM = 4; // m-tiles walked together so that concurrent workgroups share panels in L2
 
-// amdgpu_waves_per_eu(1, 1): one wavefront per SIMD is the design point (256 accumulator
+// amdgpu_waves_per_eu: from ten row tiles on one wavefront per SIMD is the design point (up to 256 accumulator
 // registers per lane); without it the register allocator chases a higher occupancy it cannot
-// reach and parks live values in the accumulator file, shuffling them around every step.
+// reach and parks live values in the accumulator file, shuffling them around every step.  Up to eight row tiles two
+// workgroups fit a CU (256 registers each, 64 KiB of LDS): one computes while the other waits at its barrier or starts a
+// tile (int8 4096 x 28672 at 333 rows, 336 workgroups of 128 rows: 120 -> 95 us; 4096 x 28672 at 160 rows, 672 of 64
+// rows on 70B gate_up: 249 -> 209 us).
 //
 // RT     row tiles (16 rows) per wavefront: the output tile is 16*RT rows x 256 columns.  16 for
-//        prefill; 8 / 4 for skinny M, where a 256-row tile would mostly multiply padding.
+//        prefill; 12 / 10 / 8 / 4 where a taller tile would mostly multiply padding (8192 x 57344 at 160 rows: 180 us
+//        with 256-row tiles, 147 with 160-row ones; 28672 x 8192 98 -> 85).
 // SPLITK several workgroups share one output tile, each covering a slice of K, and add their
 //        partial sums into a float32 buffer (skinny M x narrow N would otherwise leave most CUs idle).
 // PERSIST one workgroup per CU walks several output tiles (tile b, b + gridDim.x, ...).  The last tile
@@ -46,7 +50,7 @@ constexpr int kGemmGroupM = 4; // m-tiles walked together so that concurrent wor
 //        paid with the matrix core idle.  Plain epilogue only (bias; no activation, no residual);
 //        K must be an even number of tile rows; m * n * 2 < 2 GiB (outputs go through a descriptor).
 template <int DT, int BITS, int GROUP, bool ZERO, int RT, bool SPLITK, bool PERSIST = false, int NS_ = 4>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) gemm_kernel(GemmParams p)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 8 ? 2 : 1, RT <= 8 ? 2 : 1))) gemm_kernel(GemmParams p)
 {
     static_assert(!(PERSIST && SPLITK), "a persistent workgroup owns whole tiles");
     using E = Elem<DT>;
@@ -714,6 +718,8 @@ int launch_gemm_rt(GemmParams const& gp, int rt, hipStream_t s)
     {
     case 4: return launch_gemm_variant<DT, BITS, GROUP, ZERO, 4>(gp, s);
     case 8: return launch_gemm_variant<DT, BITS, GROUP, ZERO, 8>(gp, s);
+    case 10: return launch_gemm_variant<DT, BITS, GROUP, ZERO, 10>(gp, s);
+    case 12: return launch_gemm_variant<DT, BITS, GROUP, ZERO, 12>(gp, s);
     default:
         if (gp.tile_cols == 192)
             return launch_gemm_variant<DT, BITS, GROUP, ZERO, 16, 3>(gp, s);

@@ -28,7 +28,7 @@ inline int bits_of(int quant_type)
 
 // Experiment overrides from the environment, read once (at first use) and again by woq_reload_env():
 //   WOQ_FORCE_REGIME=stream|gemm      WOQ_STREAM_SHAPE=ns,waves,pf,lds   WOQ_WIDE_SHAPE=ns,waves,pf | 0
-//   WOQ_STREAM_SLOTS=0                WOQ_GEMM_KERNEL=exact|skinny       WOQ_GEMM_RT=4|8|16
+//   WOQ_STREAM_SLOTS=0                WOQ_GEMM_KERNEL=exact|skinny       WOQ_GEMM_RT=4|8|10|12|16
 //   WOQ_GEMM_SPLITS=<n>               WOQ_STREAM_SPLITS=<n>              WOQ_GEMM_PERSIST=0
 //   WOQ_GEMM_COLS=192|256             WOQ_ROW_SHAPE=waves,tiles | 0      WOQ_ROWS_SHAPE=waves,ns,tiles | 0
 //   WOQ_MID_SHAPE=rt,ns,waves,splits | 0
@@ -145,8 +145,12 @@ inline long gemm_tiles(int m, int n, int rt)
 //     workgroups are no faster than 192, and 257 take two rounds);
 //   * splitting K costs the reduction launch and the float32 partial slabs (written once, read once).
 // `tiles` is the output tile count of that tile height (for a grouped problem: over all experts).
-inline double gemm_cost_us(bool skinny, int rt, long tiles, int m, int n, int k, int bits, int splits, int group = -1)
+// `contract`: the estimates as they were when woq_matmul_check's workspace requirement was laid down (see plan_gemm).
+inline double gemm_cost_us(bool skinny, int rt, long tiles, int m, int n, int k, int bits, int splits, int group = -1,
+    bool contract = false)
 {
+    if (contract && group == 0)
+        group = -1;
     int const tk = tile_k_of_bits(bits);
     int const k_tiles = (k + tk - 1) / tk;
     double c;
@@ -165,7 +169,12 @@ inline double gemm_cost_us(bool skinny, int rt, long tiles, int m, int n, int k,
     int const steps = (k_tiles + splits - 1) / splits;
     double const last_round = wgs - (rounds - 1) * 32 > 28 ? 0.10 : 0.0;
     double const per_tile = skinny ? 3.15 : 1.34 + 0.081 * rt; // prologue and epilogue
-    double t = ((double) rounds + last_round) * (steps * c + per_tile) + 2.25;
+    // up to eight row tiles two workgroups of the exact kernel share a CU: a second round costs less than the first
+    // (4096 x 28672 at 333 rows, 336 workgroups of 128 rows: 120 -> 95 us against 65 for one round; 1100 rows 284 us with
+    // 256-row tiles, 234 with 128-row ones; where both pad alike the persistent 256-row kernel stays)
+    bool const fewer_rows = (m + rt * 16 - 1) / (rt * 16) * rt < (m + 255) / 256 * 16;
+    double const shared = !contract && !skinny && rt <= 8 && rounds > 1 && fewer_rows ? 0.85 : 1.0;
+    double t = ((double) rounds * shared + last_round) * (steps * c + per_tile) + 2.25;
     if (splits > 1)
         t += 2.9 + (double) m * n * 4.0 * splits * 3.3e-7;
     return t;
@@ -173,19 +182,20 @@ inline double gemm_cost_us(bool skinny, int rt, long tiles, int m, int n, int k,
 
 // The K split (1 = none) that gemm_cost_us estimates cheapest for this kernel and tile height, and
 // its cost.  A split leaves every workgroup at least four tile rows of K.
+// (`ws_limit`: bytes the float32 slabs may take.)
 inline double gemm_best_split(bool skinny, int rt, long tiles, int m, int n, int k, int bits, bool allow_split, int& splits,
-    int group = -1)
+    int group = -1, size_t ws_limit = (size_t) -1, bool contract = false)
 {
     int const tk = tile_k_of_bits(bits);
     int const k_tiles = (k + tk - 1) / tk;
     splits = 1;
-    double best = gemm_cost_us(skinny, rt, tiles, m, n, k, bits, 1, group);
+    double best = gemm_cost_us(skinny, rt, tiles, m, n, k, bits, 1, group, contract);
     if (!allow_split || k_tiles < 8)
         return best;
     for (int s = 2; s <= k_tiles / 4 && tiles * s <= 512; ++s)
     {
-        double const t = gemm_cost_us(skinny, rt, tiles, m, n, k, bits, s, group);
-        if (t < best)
+        double const t = gemm_cost_us(skinny, rt, tiles, m, n, k, bits, s, group, contract);
+        if (t < best && split_partial_bytes(m, n, s) <= ws_limit)
         {
             best = t;
             splits = s;
@@ -199,7 +209,11 @@ inline double gemm_best_split(bool skinny, int rt, long tiles, int m, int n, int
 //   * the exact-dequantize kernel with 64-, 128- or 256-row tiles.
 // Environment overrides for experiments: WOQ_GEMM_KERNEL=exact|skinny, WOQ_GEMM_RT=4|8|16 (exact
 // kernel), WOQ_GEMM_SPLITS=<n>
-inline GemmPlan plan_gemm(int m, int n, int k, int bits, bool allow_split = true, int num_experts = 1, int group = -1)
+// `ws_limit`: bytes of float32 slabs the caller brought.  `contract`: the plan whose slabs woq_matmul_check asks for.
+// What a call has to bring is part of the interface and does not move with the estimates or the tile heights: a call
+// that was accepted with some workspace stays accepted, and runs the cheapest plan that fits it.
+inline GemmPlan plan_gemm(int m, int n, int k, int bits, bool allow_split = true, int num_experts = 1, int group = -1,
+    size_t ws_limit = (size_t) -1, bool contract = false)
 {
     // rows per expert of a grouped problem (its tiles do not straddle experts)
     int const rows = num_experts > 1 ? (m + num_experts - 1) / num_experts : m;
@@ -209,17 +223,33 @@ inline GemmPlan plan_gemm(int m, int n, int k, int bits, bool allow_split = true
     GemmPlan pl{};
     double best = 0;
     bool have = false;
-    for (int cand = 0; cand < 4; ++cand)
+    // With group scales the exact kernel rounds every scaled weight to the activation type and the deferred-scale kernel
+    // none (error against 64 bits, bf16: 2.2e-3 and 1.7e-3): problems that had the latter keep it.
+    bool const deferred = !contract && group != 0 && !env.gemm_kernel
+        && plan_gemm(m, n, k, bits, allow_split, num_experts, group, ws_limit, true).skinny;
+    static constexpr int kExactRt[] = {4, 8, 10, 12, 16};
+    for (int cand = 0; cand < 6; ++cand)
     {
         bool const skinny = cand == 0;
-        int const rt = skinny ? skinny_rt : (cand == 1 ? 4 : (cand == 2 ? 8 : 16));
+        int const rt = skinny ? skinny_rt : kExactRt[cand - 1];
+        // 160- and 192-row tiles where they multiply fewer padded rows than 256-row ones (600 rows: 640 against 768)
+        if ((rt == 10 || rt == 12) && contract && !forced_rt)
+            continue;
+        if ((rt == 10 || rt == 12) && !forced_rt && (rows + rt * 16 - 1) / (rt * 16) * rt >= (rows + 255) / 256 * 16)
+            continue;
         if (env.gemm_kernel && skinny != (env.gemm_kernel == 2))
+            continue;
+        if (deferred && !skinny)
             continue;
         if (!skinny && forced_rt && rt != forced_rt)
             continue;
         int splits;
-        double const cost = gemm_best_split(
-            skinny, rt, (long) num_experts * gemm_tiles(rows, n, rt), m, n, k, bits, allow_split, splits, group);
+        long const tiles = (long) num_experts * gemm_tiles(rows, n, rt);
+        double cost = gemm_best_split(skinny, rt, tiles, m, n, k, bits, allow_split, splits, group, ws_limit, contract);
+        // the persistent form of the 256-row kernel hides its tiles' first loads and stores (6 % fewer cycles)
+        if (!contract && !skinny && rt < 16 && num_experts <= 1 && gemm_tiles(rows, n, 16) > 256
+            && (rows + rt * 16 - 1) / (rt * 16) * rt >= (rows + 255) / 256 * 16)
+            cost *= 1.07;
         if (!have || cost < best)
         {
             have = true;
