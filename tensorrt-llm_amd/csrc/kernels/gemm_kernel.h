@@ -129,22 +129,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
         for (int s = 0; s < NS; ++s)
             acc[rt][s] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // per-column scale of the per-channel mode (GROUP == 0) is loaded once
-    float pc_scale[NS];
-    uint32_t pc_scale2[NS]; // the raw 16-bit value in both halves
-    // the same for the tile row after the current one (PERSIST: another tile's columns at a tile boundary)
-    float pc_scale_n[NS];
-    uint32_t pc_scale2_n[NS];
-    if constexpr (GROUP == 0)
+    // Per-channel mode (GROUP == 0): the operands carry the bare integers - exact in either type; bf16 int4 as
+    // sixteenths, which is what the conversion instruction yields - and the column's scale multiplies the
+    // finished float32 sum: no multiply per weight, and no rounding of the scaled weight.
+    constexpr float PC_UNIT = DT == WOQ_BF16 && BITS == 4 ? 16.f : 1.f;
+    // scales of the four columns this lane holds of strip slot s (transposed accumulators)
+    auto pc_scale4 = [&](int s) -> f32x4
     {
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-        {
-            pc_scale[s] = pc_scale_n[s] = E::load(p.scales, strip_of[s] * 16 + c);
-            pc_scale2[s] = pc_scale2_n[s]
-                = (uint32_t) static_cast<uint16_t const*>(p.scales)[strip_of[s] * 16 + c] * 0x10001u;
-        }
-    }
+        u32x2 const v = *reinterpret_cast<u32x2 const*>(static_cast<uint16_t const*>(p.scales) + strip_of[s] * 16 + kg * 4);
+        return f32x4{E::lo(v[0]), E::hi(v[0]), E::lo(v[1]), E::hi(v[1])} * PC_UNIT;
+    };
+    [[maybe_unused]] f32x4 pc_store[NS] = {}; // PERSIST: those of the tile whose outputs are stored next
 
     // A tile -> LDS.  Fragment f = rt * SLABS + j is 1 KiB: the 16 rows x 32 k that one MFMA
     // consumes.  The DMA writes lane l's 16 bytes at offset l*16 of the fragment, so the lane
@@ -246,7 +241,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
     constexpr int A_AHEAD = 3;
     u32x4 b_cur[NS], b_nxt[NS];
 
-    auto scale_of = [&](BStage const& st, int s, int seg, float& sc, float& zr, bool next_step = false)
+    auto scale_of = [&](BStage const& st, int s, int seg, float& sc, float& zr)
     {
         if constexpr (GROUP != 0)
         {
@@ -255,13 +250,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
         }
         else
         {
-            sc = next_step ? pc_scale_n[s] : pc_scale[s];
+            sc = 1.f / PC_UNIT;
             zr = 0.f;
         }
     };
 
     // the same as packed half-precision pairs (s, s) and (z, z), from the raw 16-bit values
-    auto scale_pair_of = [&](BStage const& st, int s, int seg, uint32_t& s2, uint32_t& z2, bool next_step = false)
+    auto scale_pair_of = [&](BStage const& st, int s, int seg, uint32_t& s2, uint32_t& z2)
     {
         if constexpr (GROUP != 0)
         {
@@ -269,10 +264,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
             z2 = ZERO ? (uint32_t) st.z[s][seg] * 0x10001u : 0u;
         }
         else
-        {
-            s2 = next_step ? pc_scale2_n[s] : pc_scale2[s];
-            z2 = 0u;
-        }
+            s2 = z2 = 0u;
     };
 
     // PERSIST: where the finished tile's outputs go (set when the workgroup moves on to its next tile)
@@ -290,7 +282,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[r]) : "a"(acc[rt][s][r]));
-        u32x2 const o = {E::pack(p.alpha * v[0], p.alpha * v[1]), E::pack(p.alpha * v[2], p.alpha * v[3])};
+        f32x4 const f = GROUP == 0 ? pc_store[s] * p.alpha : f32x4{p.alpha, p.alpha, p.alpha, p.alpha};
+        u32x2 const o = {E::pack(f[0] * v[0], f[1] * v[1]), E::pack(f[2] * v[2], f[3] * v[3])};
         // the row-tile offset belongs in the vector offset: the descriptor's range check does not
         // see the scalar offset, and rows past M must be dropped by it
         __builtin_amdgcn_raw_buffer_store_b64(o, out_rsrc, (int) (prev_off + (uint32_t) rt * rt_stride + (uint32_t) s * 32u), 0, 0);
@@ -355,7 +348,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                         {
                             if (stage == 0)
                             {
-                                scale_of(src, s, jn / SEG_SLABS, sc[x], zr[x], !same_step);
+                                scale_of(src, s, jn / SEG_SLABS, sc[x], zr[x]);
                                 sc[x] *= BITS == 4 ? 16.f : 1.f;
                             }
                             else if (stage == 1)
@@ -367,8 +360,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                             }
                             else if (stage == 2)
                             {
-                                t0[x] = __builtin_fmaf(t0[x], sc[x], zr[x]);
-                                t1[x] = __builtin_fmaf(t1[x], sc[x], zr[x]);
+                                if constexpr (GROUP != 0)
+                                {
+                                    t0[x] = __builtin_fmaf(t0[x], sc[x], zr[x]);
+                                    t1[x] = __builtin_fmaf(t1[x], sc[x], zr[x]);
+                                }
                             }
                             else
                                 b_nxt[s][pr] = E::pack(t0[x], t1[x]);
@@ -376,7 +372,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                         else
                         {
                             if (stage == 0)
-                                scale_pair_of(src, s, jn / SEG_SLABS, s2[x], z2[x], !same_step);
+                                scale_pair_of(src, s, jn / SEG_SLABS, s2[x], z2[x]);
                             else if (stage == 1)
                             {
                                 if constexpr (BITS == 4)
@@ -387,7 +383,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                             else if (stage == 2)
                                 h2[x] = half2_add(h2[x], -Offset<DT, BITS>::value);
                             else
-                                b_nxt[s][pr] = half2_fma(h2[x], s2[x], z2[x]);
+                                b_nxt[s][pr] = GROUP != 0 ? half2_fma(h2[x], s2[x], z2[x]) : h2[x];
                         }
                     }
                 };
@@ -473,6 +469,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
             step_barrier();
             compute(std::true_type{}, a_buf0, st0, st1, a_buf1, 1);
             step_barrier();
+            if constexpr (GROUP == 0)
+            {
+                // the previous tile's outputs are out: from here on the scales of this tile's columns
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    pc_store[s] = pc_scale4(s);
+            }
             compute(std::false_type{}, a_buf1, st1, st0, a_buf0, 2);
             for (int kt = 2; kt < KT - 2; kt += 2)
             {
@@ -499,12 +502,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                             strip_of[s] = paired_strip(false, strip0, s, p.strips, strip_ok[s]);
                             wlane[s] = ((uint32_t) strip_of[s] * (uint32_t) p.k_tiles * 64u + (uint32_t) lane) * 16u;
                             sc_lane[s] = (uint32_t) (strip_of[s] * 16 + c) * 2u;
-                            if constexpr (GROUP == 0)
-                            {
-                                pc_scale_n[s] = E::load(p.scales, strip_of[s] * 16 + c);
-                                pc_scale2_n[s]
-                                    = (uint32_t) static_cast<uint16_t const*>(p.scales)[strip_of[s] * 16 + c] * 0x10001u;
-                            }
                         }
                         dma_lane_base = ((uint32_t) (m0 + (wave / SLABS) * 16 + (lane >> 2)) * (uint32_t) K
                                             + (uint32_t) (dma_j * 32 + (((lane & 3) ^ frag_swizzle(lane >> 4)) * 8)))
@@ -514,15 +511,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                         tile_oob = kOob;
                 }
                 compute(std::false_type{}, a_buf1, st1, st0, a_buf0, 0);
-            }
-            if constexpr (GROUP == 0)
-            {
-#pragma unroll
-                for (int s = 0; s < NS; ++s)
-                {
-                    pc_scale[s] = pc_scale_n[s];
-                    pc_scale2[s] = pc_scale2_n[s];
-                }
             }
         } while (!tile_oob);
         // the last tile's outputs
@@ -542,6 +530,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
         // plain orientation: acc[rt][s][r] = (row m0 + rt*16 + kg*4 + r, column strip*16 + c);
         // this K slice's own slab of the partial buffer (a slice past the end of K stores zeros)
         float* const slab = p.partial + (size_t) blockIdx.y * ((size_t) p.m * p.n);
+        [[maybe_unused]] float pc[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            pc[s] = GROUP == 0 ? E::load(p.scales, strip_of[s] * 16 + c) * PC_UNIT : 1.f;
 #pragma unroll
         for (int s = 0; s < NS; ++s)
 #pragma unroll
@@ -551,7 +543,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                 {
                     int const row = m0 + rt * 16 + kg * 4 + r;
                     if (strip_ok[s] && row < p.m)
-                        slab[(size_t) row * p.n + strip_of[s] * 16 + c] = acc[rt][s][r];
+                        slab[(size_t) row * p.n + strip_of[s] * 16 + c] = GROUP == 0 ? acc[rt][s][r] * pc[s] : acc[rt][s][r];
                 }
         return;
     }
@@ -594,12 +586,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                 constexpr bool RESIDUAL = decltype(residual_tag)::value;
                 int col[NS / 2];
                 f32x4 bias_x[NS / 2], bias_g[NS / 2];
+                [[maybe_unused]] f32x4 pc_x[NS / 2], pc_g[NS / 2];
 #pragma unroll
                 for (int i = 0; i < NS / 2; ++i)
                 {
                     col[i] = strip_of[2 * i] * 16 + kg * 4; // strip_of[even slot] is the pair index (value half)
                     bias_x[i] = p.bias ? load4(p.bias, col[i]) : zero4;
                     bias_g[i] = p.bias ? load4(p.bias, col[i] + n_out) : zero4;
+                    if constexpr (GROUP == 0)
+                        pc_x[i] = pc_scale4(2 * i), pc_g[i] = pc_scale4(2 * i + 1);
                 }
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
@@ -617,8 +612,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                         f32x4 v;
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
-                            v[r] = (acc[rt][2 * i][r] + bias_x[i][r]) * apply_act(ACT, acc[rt][2 * i + 1][r] + bias_g[i][r])
-                                + res[i][r];
+                        {
+                            float x = acc[rt][2 * i][r], g = acc[rt][2 * i + 1][r];
+                            if constexpr (GROUP == 0)
+                                x *= pc_x[i][r], g *= pc_g[i][r];
+                            v[r] = (x + bias_x[i][r]) * apply_act(ACT, g + bias_g[i][r]) + res[i][r];
+                        }
                         store4(row, col[i], v);
                     }
                 }
@@ -641,6 +640,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
         col[s] = strip_of[s] * 16 + kg * 4;
         bias[s] = (!SPLITK && p.bias) ? load4(p.bias, col[s]) : zero4;
     }
+    [[maybe_unused]] f32x4 pc[NS];
+    if constexpr (GROUP == 0)
+    {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            pc[s] = pc_scale4(s);
+    }
     auto plain_epilogue = [&](auto residual_tag)
     {
     constexpr bool RESIDUAL = decltype(residual_tag)::value;
@@ -660,7 +666,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
             f32x4 v;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                v[r] = __builtin_fmaf(p.alpha, acc[rt][s][r], bias[s][r]) + res[s][r];
+                v[r] = __builtin_fmaf(GROUP == 0 ? p.alpha * pc[s][r] : p.alpha, acc[rt][s][r], bias[s][r]) + res[s][r];
             store4(row, col[s], v);
         }
     }

@@ -157,9 +157,14 @@ inline double gemm_cost_us(bool skinny, int rt, long tiles, int m, int n, int k,
     if (skinny)
         // (two row tiles: 0.79 before the A fragments were read a step ahead; four row tiles at group size 128:
         // 1.19 before the fragments were read just in time and placed free of LDS bank conflicts, re-measured
-        // against the exact-dequantize kernel at 48 ... 128 rows since - `group` is -1 where the caller does not
+        // against the exact-dequantize kernel at 48 ... 128 rows since; per-channel scales, which leave nothing to
+        // apply per step: 0.80 / 0.47, from eight experts of 14336 x 4096 - `group` is -1 where the caller does not
         // know it)
-        c = bits == 4 ? (rt == 2 ? 0.73 : (group == 128 ? 1.03 : 1.29)) : 0.565;
+        c = bits == 4 ? (rt == 2 ? (group == 0 ? 0.47 : 0.73) : (group == 128 ? 1.03 : (group == 0 ? 0.80 : 1.29))) : 0.565;
+    else if (group == 0)
+        // (bare integers as operands, the scale in the epilogue: 4096 x 28672 at 64 / 128 / 333 rows 34.4 / 48.9 / 74
+        // and, int8, 58 / 65 / 80 us on 4-, 8- and 12-row-tile kernels)
+        c = bits == 4 ? 0.50 + 0.113 * rt : 0.62 + 0.0375 * rt;
     else
         c = bits == 4 ? 0.807 + 0.108 * rt : 0.642 + 0.0404 * rt;
     // the tiles are dealt to the 8 XCDs (32 CUs each) in equal contiguous runs: the fullest XCD
@@ -244,7 +249,13 @@ inline GemmPlan plan_gemm(int m, int n, int k, int bits, bool allow_split = true
         if (!skinny && forced_rt && rt != forced_rt)
             continue;
         int splits;
-        long const tiles = (long) num_experts * gemm_tiles(rows, n, rt);
+        // row tiles of a grouped problem: an expert's last tile is half full on average, and one it has at least
+        // (rows per expert differ: rounding the average up to whole tiles took 128-row tiles for 75 rows on average,
+        // 43 ... 119 in fact, where 64-row tiles run fewer)
+        double const expected = (double) m / (16.0 * rt) + 0.5 * num_experts;
+        long const tiles = num_experts <= 1 || contract
+            ? (long) num_experts * gemm_tiles(rows, n, rt)
+            : (long) (expected > num_experts ? expected : num_experts) * ((n + 255) / 256);
         double cost = gemm_best_split(skinny, rt, tiles, m, n, k, bits, allow_split, splits, group, ws_limit, contract);
         // the persistent form of the 256-row kernel hides its tiles' first loads and stores (6 % fewer cycles)
         if (!contract && !skinny && rt < 16 && num_experts <= 1 && gemm_tiles(rows, n, 16) > 256
