@@ -57,6 +57,36 @@ GemmPlan planned_gemm(int m, int n, int k, int bits, int group, size_t ws_limit 
     return plan_gemm(m, n, k, bits, true, 1, group, ws_limit, contract);
 }
 
+bool pick_rows_shape(int m, int n, int k, int group, int bits, bool pqs, int& waves, int& ns, int& tiles);
+
+// The same kernel with one row tile, for up to sixteen rows of int4 weights that the multi-row kernel leaves to the staged
+// one, whose activation fragments come straight into registers (quads of lanes read four rows: a quarter of the L1's
+// rate), so that its time grows with the rows.  Measured against it (us, staged -> this): group 64 at 16 rows, 8192 x 57344
+// 53.4 -> 51.0, 8192 x 10240 17.3 -> 14.2, 28672 x 8192 29.4 -> 28.4, 8192 x 8192 12.0 -> 10.8; group 128 at 12 / 16 rows,
+// 8192 x 57344 46.0 -> 45.1 / 48.7 -> 47.2, 8192 x 10240 13.4 -> 12.7 / 14.0 -> 13.4, 4096 x 28672 14.4 -> 14.1 / 15.2 ->
+// 14.6; per-channel at 8 / 16 rows, 4096 x 4096 6.3 -> 5.2 / 7.4 -> 5.8, 8192 x 8192 9.4 -> 9.0 / 11.6 -> 10.2.  Fewer rows:
+// even or slower, but for group 64 on 513 ... 1024 strips (8 rows 17.0 -> 13.3).  int8: no gain.
+bool pick_mid_one_tile(MatmulProblem const& p, MidPlan& plan)
+{
+    EnvOverrides const& env = env_overrides();
+    int waves, ns, tiles;
+    int const strips = p.n / kTileN;
+    int const from = p.group_size == 0 || (p.group_size == 64 && strips > 512 && strips <= 1024) ? 8 : 12;
+    if (p.bits != 4 || p.m < from || p.k < 2048 || env.rows_mode != -1 || env.row_mode != -1 || env.wide_mode != -1
+        || env.slots_off || pick_rows_shape(p.m, p.n, p.k, p.group_size, p.bits, false, waves, ns, tiles))
+        return false;
+    if (p.k >= 8192 && p.k >= 2 * p.n) // the down projections: too few strips for whole-K workgroups
+    {
+        plan = strips <= 256 ? MidPlan{1, 4, 8, 4} : MidPlan{1, 4, 4, 4};
+        return p.workspace && split_partial_bytes(p.m, p.n, plan.splits) <= p.workspace_bytes;
+    }
+    plan = strips <= 256 ? MidPlan{1, 1, 8, 1}
+        : strips <= 512  ? MidPlan{1, 2, 8, 1}
+        : strips <= 1024 ? MidPlan{1, 4, 8, 1}
+                         : MidPlan{1, 4, 4, 1};
+    return true;
+}
+
 // The barrier-free mid-M kernel (mid_kernel.h) for this problem, and its launch shape: where mid_cost_us estimates it
 // cheaper than `other_us`, the estimate of the kernel the regime would run.  Measured against those (bf16, group 128,
 // zeros; us, old -> new): 4096 x 4096 at 32 / 48 / 64 / 96 / 160 rows 10.5 -> 7.9 / 14.2 -> 9.6 / 15.7 -> 10.2 / 18.7 ->
@@ -74,8 +104,10 @@ bool pick_mid_shape(MatmulProblem const& p, double other_us, MidPlan& plan)
         plan = MidPlan{env.mid_shape[0], env.mid_shape[1], env.mid_shape[2], env.mid_shape[3]};
         return true;
     }
-    if (!p.built_in_choice || p.m <= 16 || p.m > kMidMaxM)
+    if (!p.built_in_choice || p.m > kMidMaxM)
         return false;
+    if (p.m <= 16)
+        return pick_mid_one_tile(p, plan);
     double const t = best_mid_plan(p.m, p.n, p.k, p.bits, p.group_size, p.workspace ? p.workspace_bytes : 0, plan);
     // (0.88: with the two models' errors, 3 of 95 measured problems end up slower than before, by 1 ... 7 %, and the choice
     // costs 2 % on average against the better of the two; at 1.0 a few lose 10 % and the average gains nothing)

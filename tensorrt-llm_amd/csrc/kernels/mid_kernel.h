@@ -1,4 +1,4 @@
-// 17 to 160 rows without a barrier in the main loop: the rows between the decode kernels and the tall prefill tiles
+// 8 to 160 rows without a barrier in the main loop: the rows between the decode kernels and the tall prefill tiles
 // (the reference covers them with CUTLASS tiles of 16 ... 64 rows and split-K,
 // cpp/tensorrt_llm/kernels/cutlass_kernels/cutlass_heuristic.cpp:59-140).
 //
@@ -25,7 +25,7 @@
 // on 4096 x 28672 take 19 instead of 24 us), where the tiled kernels' 256 columns win from 64 rows on.
 // Measured (bf16, group 128, zeros; before -> now, us): 4096 x 4096 at 32 / 48 / 64 / 160 rows 10.5 -> 7.9 / 14.2 -> 9.6 /
 // 15.7 -> 10.2 / 20.8 -> 13.6; 4096 x 6144 at 48 rows 16.0 -> 10.7; 8192 x 8192 at 48 rows 19.2 -> 17.2; 4096 x 28672 at
-// 48 rows 27.5 -> 23.7 (2.6 TB/s of weights).
+// 48 rows 27.5 -> 23.7 (2.6 TB/s of weights); group 64, 8192 x 10240 at 16 rows 17.3 -> 14.2.
 // Needs k to be a multiple of the weight tile's rows (128 for int4, 64 for int8).
 #pragma once
 
@@ -411,6 +411,10 @@ int launch_mid_shaped(MatmulProblem const& p, MidPlan const& plan, hipStream_t s
     {                                                                                                                  \
         WOQ_MID(RT_, 4, 4)                                                                                             \
         WOQ_MID(RT_, 4, 8)                                                                                             \
+    }
+    if constexpr (BITS == 4) // (int8: the other streaming kernels are as fast)
+    {
+        WOQ_MID_RT(1)
     }
     WOQ_MID_RT(2)
     WOQ_MID_RT(3)

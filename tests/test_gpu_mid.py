@@ -19,13 +19,15 @@ def _instantiated(rt, ns, group):
     return group == 0 or ns < 4 or rt < (3 if group == 64 else 4)
 
 
-@pytest.mark.parametrize("rt", [2, 3, 4])
+@pytest.mark.parametrize("rt", [1, 2, 3, 4])
 @pytest.mark.parametrize("bits,group,dtype", [(4, 128, "bf16"), (4, 64, "fp16"), (4, 0, "bf16"), (8, 0, "fp16"),
                                               (8, 0, "bf16"), (4, 128, "fp16"), (4, 64, "bf16")])
 def test_mid_every_shape(pkg, oracle, dev, woq_env, rt, bits, group, dtype):
     """Strips that do not divide by a workgroup's, one row past a row tile / a whole tile / a second tile of rows, tile
     rows of K that leave some wavefronts one more than others (or none), K split with a last slice that is shorter;
     zeros, bias and smoothing on and off; the same bits on every call."""
+    if rt == 1 and bits == 8:
+        pytest.skip("one row tile is built for int4 only")
     tk = 128 if bits == 4 else 64
     for ns, waves in SHAPES:
         if not _instantiated(rt, ns, group):
@@ -71,15 +73,18 @@ def test_mid_against_the_general_path(pkg, oracle, dev, woq_env, bits, group):
 
 
 def test_mid_rule(pkg, oracle, dev, woq_env):
-    """Taken on narrow matrices from 17 rows on when nothing is forced; not for one row tile, wide matrices at 64 rows,
-    flexible groups, int8 with group scales, a K that is no multiple of the weight tile, or a regime the caller named."""
+    """Taken on narrow matrices from 17 rows on when nothing is forced; with one row tile where the multi-row kernel
+    declines; not for more than 160 rows, flexible groups, int8 with group scales, a K that is no multiple of the weight
+    tile, a smoothing vector that the streaming regime would apply itself, or a regime the caller named."""
     woq_env(WOQ_MID_SHAPE=None)
     run = lambda M, K, N, bits, group, regime=0: (run_product(
         pkg, oracle, dev, random_problem(oracle, M, K, N, bits, group, "bf16", seed=M), regime), _last_launch(pkg))[1]
     for M in (17, 33, 48, 64, 65, 160):
         assert "mid" in run(M, 4096, 1024, 4, 128), M
     assert "mid" in run(48, 4096, 1024, 8, 0)
-    for args in [(16, 4096, 1024, 4, 128), (161, 4096, 1024, 4, 128), (48, 4096, 1024, 4, 256), (48, 4096, 1024, 8, 128),
+    assert "mid rt=1" in run(16, 2048, 8208, 4, 128) and "mid rt=1" in run(8, 2048, 1024, 4, 0)
+    assert "mid rt=1 ns=4 waves=8 splits=4" in run(12, 8192, 272, 4, 64)
+    for args in [(16, 4096, 1024, 4, 128), (11, 2048, 8208, 4, 128), (16, 2048, 1024, 8, 0), (161, 4096, 1024, 4, 128), (48, 4096, 1024, 4, 256), (48, 4096, 1024, 8, 128),
                  (48, 2112, 1024, 4, 64)]:
         assert "mid" not in run(*args), args
     for regime in (1, 2):
