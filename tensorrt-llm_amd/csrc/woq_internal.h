@@ -261,6 +261,10 @@ inline GemmPlan plan_gemm(int m, int n, int k, int bits, bool allow_split = true
         if (!contract && !skinny && rt < 16 && num_experts <= 1 && gemm_tiles(rows, n, 16) > 256
             && (rows + rt * 16 - 1) / (rt * 16) * rt >= (rows + 255) / 256 * 16)
             cost *= 1.07;
+        // experts differ in their rows, and a tall tile multiplies the rows it does not have (eight experts of 4096 x 28672,
+        // 43 ... 119 rows: 206 us with 64-row tiles, 235 with 128-row ones that the bare count ranks first)
+        if (!contract && !skinny && rt > 4 && num_experts > 1)
+            cost *= 1.12;
         if (!have || cost < best)
         {
             have = true;
