@@ -96,7 +96,8 @@ bool pick_mid_one_tile(MatmulProblem const& p, MidPlan& plan)
 bool pick_mid_shape(MatmulProblem const& p, double other_us, MidPlan& plan)
 {
     EnvOverrides const& env = env_overrides();
-    if (env.mid_mode == 0 || p.w4a8 || p.pre_quant_scale || p.num_experts || p.activation != WOQ_ACT_IDENTITY || p.residual
+    // (activations that do not start on 16 bytes stay with kernels that load them to registers: the DMA moves 16-byte pieces)
+    if (env.mid_mode == 0 || reinterpret_cast<uintptr_t>(p.act) % 16 || p.w4a8 || p.pre_quant_scale || p.num_experts || p.activation != WOQ_ACT_IDENTITY || p.residual
         || p.k % tile_k_of_bits(p.bits) || (p.group_size != 0 && (p.bits == 8 || p.group_size > 128)))
         return false;
     if (env.mid_mode == 1)
@@ -981,8 +982,10 @@ static int run_matmul(const woq_matmul_args* args, void* stream)
     if (p.m == 0)
         return WOQ_OK;
     EnvOverrides const& env = env_overrides();
-    p.built_in_choice = args->regime == WOQ_REGIME_AUTO && env.regime == WOQ_REGIME_AUTO && !current_tactic()
-        && !env.gemm_kernel && !env.gemm_rt && !env.gemm_splits && !env.has_stream_shape && !env.stream_splits;
+    Tactic const* const tactic = current_tactic(); // one of regime AUTO is the tuned table's "as the heuristics choose"
+    p.built_in_choice = args->regime == WOQ_REGIME_AUTO && env.regime == WOQ_REGIME_AUTO
+        && (!tactic || tactic->regime == WOQ_REGIME_AUTO) && !env.gemm_kernel && !env.gemm_rt && !env.gemm_splits
+        && !env.has_stream_shape && !env.stream_splits;
     bool const streaming = pick_regime(args) == WOQ_REGIME_STREAM;
     if (streaming && !p.w4a8)
         return launch_stream(p, stream); // smoothing is fused into the 16-bit streaming kernel

@@ -91,6 +91,39 @@ def test_mid_rule(pkg, oracle, dev, woq_env):
         assert "mid" not in run(48, 4096, 1024, 4, 128, regime)
 
 
+def test_mid_needs_aligned_activations(pkg, oracle, dev, woq_env):
+    """Activations that start 8 bytes into an allocation run on the kernel that took them before, with the same result."""
+    from _util import preprocess, to_dev
+    F = pkg.functional
+    woq_env(WOQ_MID_SHAPE=None)
+    p = random_problem(oracle, 32, 4096, 1024, 4, 128, "bf16", seed=4)
+    w, sc = preprocess(pkg, oracle, p["q"], 4).to(dev), to_dev(p["scales"], "bf16", dev)
+    room = torch.empty(32 * 4096 + 8, dtype=torch.bfloat16, device=dev)
+    for skip, mid in ((8, True), (4, False)):
+        act = room[skip:skip + 32 * 4096].view(32, 4096)
+        act.copy_(to_dev(p["act"], "bf16", dev))
+        out = F.woq_matmul_raw(act, None, w, sc, None, None, n=1024, k=4096, group_size=128, quant_algo=0)
+        torch.cuda.synchronize()
+        assert ("mid" in _last_launch(pkg)) == mid, _last_launch(pkg)
+        assert parity_err(oracle, out.float().cpu().numpy(), p) < TOL
+
+
+def test_mid_and_the_tuned_table(pkg, oracle, dev, woq_env):
+    """A table entry that leaves the choice to the heuristics leaves this kernel in it; one that names another does not."""
+    F = pkg.functional
+    woq_env(WOQ_MID_SHAPE=None)
+    p = random_problem(oracle, 48, 4096, 1024, 4, 128, "bf16", seed=3)
+    key = "1024 4096 0 128 %d 48 " % F._WOQ_DT[torch.bfloat16]
+    try:
+        for entry, mid in (("0 0 0 0 0 0 0 0 0", True), ("2 0 0 0 0 0 0 4 2", False)):
+            F.import_tactics("woq-tactics 1\n" + key + entry + "\n")
+            out = run_product(pkg, oracle, dev, p, 0)
+            assert ("mid" in _last_launch(pkg)) == mid, _last_launch(pkg)
+            assert parity_err(oracle, out, p) < TOL
+    finally:
+        F.clear_tactics()
+
+
 def test_mid_split_only_with_room(pkg, oracle, dev, woq_env):
     """A long K on few columns splits K when the workspace holds the slabs and runs without a split otherwise."""
     F = pkg.functional
