@@ -11,6 +11,7 @@ namespace woq
 {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -61,6 +62,17 @@ struct Elem<WOQ_BF16>
     static __device__ __forceinline__ void mma_first(u32x4 a, u32x4 b, f32x4& c)
     {
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
+    }
+
+    // the same on blocks of 32 x 32 x 16: twice the work for one issue slot
+    static __device__ __forceinline__ void mma_acc(u32x4 a, u32x4 b, f32x16& c)
+    {
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    }
+
+    static __device__ __forceinline__ void mma_first(u32x4 a, u32x4 b, f32x16& c)
+    {
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
     }
 
     static __device__ __forceinline__ float lo(uint32_t pair)
@@ -126,6 +138,17 @@ struct Elem<WOQ_FP16>
         asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
     }
 
+    // the same on blocks of 32 x 32 x 16: twice the work for one issue slot
+    static __device__ __forceinline__ void mma_acc(u32x4 a, u32x4 b, f32x16& c)
+    {
+        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    }
+
+    static __device__ __forceinline__ void mma_first(u32x4 a, u32x4 b, f32x16& c)
+    {
+        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
+    }
+
     static __device__ __forceinline__ float lo(uint32_t pair)
     {
         return (float) bit_cast<f16x2>(pair)[0];
@@ -171,6 +194,13 @@ struct Elem<WOQ_FP16>
 __device__ __forceinline__ void mma_drain()
 {
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+}
+
+// The same without holding back memory operations, for inside a main loop: 20 wait states, one more than a vector
+// instruction needs behind a 16-pass matrix instruction.
+__device__ __forceinline__ void mma_settle()
+{
+    asm volatile("s_nop 15\n\ts_nop 3");
 }
 
 // ---- packed weights -> MFMA B operand holding (BASE + u) exactly ---------------------------

@@ -8,20 +8,25 @@
 // multiples (the reference's pre-Hopper launcher takes 128 only, fpA_intB_gemm_template.h:136-142; its
 // Hopper launcher any multiple of the K tile, launchers/fpA_intB_launcher_sm90.inl:190-198).
 //
-// Same skeleton as the 16-bit prefill kernel (gemm_kernel.h): output tile 16*RT rows x 256
-// columns, 4 wavefronts side by side along N with 64 columns each; packed weights go global ->
-// registers and are dequantized once per workgroup; the activation tile is DMA-ed
-// global -> LDS, double-buffered; the requests of the next step and the conversions are spread
-// between the MFMAs; skinny problems split K through the float32 partial buffer.
-// The matrix instruction is the CDNA4 v_mfma_f32_16x16x128_f8f6f4 (e4m3 x e4m3): one instruction
-// covers a whole 128-deep tile row, twice the rate of the 16x16x32 fp8 form and a quarter of its
-// issue slots.  A lane supplies 32 k-values of its row / column; which 32 is free as long as A
-// and B agree, so lane (kg, c) keeps the tile layout's own order - its 8 weights of slab 0, of
-// slab 1, ... (k = 32 j + 8 kg + e) - and reads the matching four 8-byte pieces of its activation
-// row from LDS.
+// Output tile 16*RT rows x 256 columns, 8 wavefronts side by side along N with 32 columns each (two a SIMD: one issues
+// under the other's waits); packed weights go global -> registers and are dequantized once per workgroup, between the
+// MFMAs; the activation tile is DMA-ed global -> LDS; skinny problems split K through the float32 partial buffer.
+// Requests run three steps of 128 rows of K ahead, into four LDS buffers and register stages: a wavefront waits for
+// nothing it requested less than two steps ago, and reads the next step's first operands before the barrier.
+// The matrix instruction is the CDNA4 v_mfma_f32_32x32x64_f8f6f4 (e4m3 x e4m3): twice the work of a 16x16x128 one for an
+// issue slot.  A lane supplies 32 k-values of its row / column; which 32 is free as long as A
+// and B agree: lane (kh, row) takes the 16 values 32 j + 16 kh ... of two slabs j, two neighbouring chunks of the weight
+// layout and one 16-byte read of the activations each.
 // An fp8 activation fragment is half the size of a 16-bit one, so LDS holds fragment PAIRS: 16
 // rows x 64 k = 1 KiB, written by one DMA instruction (lane 4r+q fetches row r's 16-byte chunk
-// q ^ (r>>2): quads read 64 contiguous bytes, the XOR spreads an MFMA lane group over the banks).
+// q ^ (r>>2): quads read 64 contiguous bytes, the XOR spreads the reads of a block's rows over the banks).
+// Measured (bf16 output, group 128, no zero-points, us; before: four wavefronts of 64 columns, 16x16x128 instructions,
+// two buffers, arithmetic conversion): 4096 x 28672 at 64 / 1990 / 8192 rows 55.9 -> 26.8 / 234 -> 198 / 851 -> 737 (2.61
+// PFLOP/s), 8192 x 57344 at 128 / 256 rows 119 -> 69.6 / 116 -> 107, 4096 x 4096 at 1990 rows 54.3 -> 36.2 (128-row tiles).
+// By step, 8192 x 57344 at 128 rows: 32x32x64 109, eight wavefronts 88, three steps ahead 75, look-up conversion 70.
+// What bounds it: 128-row tiles the conversions (140 issue slots of each wavefront a step beside 8 instructions of 64
+// cycles); 256-row ones the LDS (every wavefront reads the whole activation tile: 2048 + 256 cycles a step, as many as the
+// matrix core is busy) and, at 8192 rows, the clock.
 #include "gemm_common.h"
 #include "w4a8_common.h"
 
@@ -35,20 +40,28 @@ namespace woq
 // block's new sum.  The 8 us or so that a tile spends outside its main loop (first loads, the
 // conversion of the first operand set, 128 KiB of stores, the relaunch) weigh twice as much here as
 // there: a tile's main loop is half as long.
-template <int ODT, bool ZERO, int RT, bool SPLITK, bool PERSIST = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) gemm_w4a8_kernel(GemmParams p)
+constexpr int kW4a8Waves = 8;
+constexpr int kOneTile = 0, kPersistPairs = 1, kPersist = 2; // persistent forms: steps in pairs (any even K), in fours
+
+template <int ODT, bool ZERO, int RT, bool SPLITK, int LOOP = kOneTile>
+__global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm_w4a8_kernel(GemmParams p)
 {
+    constexpr bool PERSIST = LOOP != kOneTile, DEEP = LOOP != kPersistPairs;
+    constexpr int NW = kW4a8Waves;
     static_assert(!PERSIST || (RT == 16 && !SPLITK && ODT == WOQ_BF16), "persistent form: 256-row tiles, whole K, bf16 out");
     using EO = Elem<ODT>;
-    using EH = Elem<WOQ_FP16>;
-    constexpr int TK = 128, SLABS = 4, NS = 4;
+    constexpr int TK = 128, NS = 16 / NW;
     constexpr int BM = RT * 16;
+    constexpr int BLK = 32, RB = BM / BLK, CB = NS * 16 / BLK; // 32 x 32 blocks of a wavefront along M and N
+    constexpr int KI = TK / 64;                                // matrix instructions along a tile row
     constexpr int PAIRS = RT * 2;      // fragment pairs (1 KiB) of one A tile
     constexpr int A_BYTES = BM * TK;   // e4m3: one byte per element
-    static_assert(PAIRS % 4 == 0, "fragment pairs spread evenly over the 4 wavefronts");
+    static_assert(PAIRS % NW == 0 && CB == 1, "one column block a wavefront; fragment pairs spread evenly over the wavefronts");
 
     __shared__ u32x4 a_buf0[A_BYTES / 16];
     __shared__ u32x4 a_buf1[A_BYTES / 16];
+    __shared__ u32x4 a_buf2[A_BYTES / 16];
+    __shared__ u32x4 a_buf3[A_BYTES / 16];
 
     // Tile of virtual block vb (the block index, or with PERSIST the block index plus a multiple of the
     // grid size, which is a multiple of 8): XCD-contiguous chunks of the tile order, m fastest inside
@@ -58,16 +71,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     int const per_xcd = (total + 7) / 8;
     auto tile_of = [&](int vb, int& tm_, int& tn_) -> bool
     {
-        int const t = (vb & 7) * per_xcd + (vb >> 3);
-        if ((vb >> 3) >= per_xcd || t >= total)
-            return false;
+        int t = (vb & 7) * per_xcd + (vb >> 3);
+        bool const exists = (vb >> 3) < per_xcd && t < total;
+        t = exists ? t : 0; // (no branch: the persistent loop's registers do not survive one between its steps)
         constexpr int kGroupM = 4;
         int const in_group = kGroupM * p.tiles_n;
         int const first_m = (t / in_group) * kGroupM;
         int const gsz = p.tiles_m - first_m < kGroupM ? p.tiles_m - first_m : kGroupM;
         tm_ = first_m + (t % in_group) % gsz;
         tn_ = (t % in_group) / gsz;
-        return true;
+        return exists;
     };
     int vb = (int) blockIdx.x;
     int tm, tn;
@@ -76,7 +89,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int const c = lane & 15, kg = lane >> 4;
+    int const row_in = lane & 31, kh = lane >> 5; // row of a block, half of K that the lane feeds
     int const K = p.k;
     int const kt_begin = SPLITK ? (int) blockIdx.y * p.tiles_per_split : 0;
     int const KT = SPLITK ? (kt_begin + p.tiles_per_split < p.k_tiles ? kt_begin + p.tiles_per_split : p.k_tiles)
@@ -87,7 +100,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     constexpr uint32_t kOob = 0x80000000u;
     auto const act_rsrc = make_rsrc(p.act, (uint32_t) p.m * (uint32_t) K);
     uint32_t const sz_bytes = (uint32_t) p.scale_rows * (uint32_t) p.n * 2u;
-    uint32_t const magic = p.group_magic; // groups above 128: table row of a tile row (w4a8_scale_row)
+    // table row of tile row kt (w4a8_scale_row) without its case distinction, which becomes a branch in the persistent
+    // loop: kt itself for groups of 128, else kt / (group / 128), as the upper half of 2 kt * ceil(2^31 / (group / 128))
+    uint32_t const magic = p.group_magic ? (p.group_magic >> 1) + (p.group_magic & 1u) : 0x80000000u;
     auto const sc_rsrc = make_rsrc(p.scales, sz_bytes);
     auto const zr_rsrc = make_rsrc(ZERO ? p.zeros : p.scales, sz_bytes);
     auto const w_rsrc = make_rsrc(p.weight, (uint32_t) p.strips * (uint32_t) p.k_tiles * 1024u);
@@ -95,20 +110,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     // per-lane request addresses of one tile (PERSIST keeps those of the next tile beside them)
     struct TileCtx
     {
-        uint32_t wlane[NS], sc_lane[NS];
+        uint32_t wlane[CB], sc_lane[CB]; // column blocks of two strips; chunks 2 kh and 2 kh + 1 of the lane's column
         uint32_t dma_lane_base;
         uint32_t oob; // kOob: there is no such tile, every request reads zeros
     };
+    // Which weight column a lane feeds to row row_in of its block is free.  A block's sums come back with lane
+    // (kh, row_in) holding operand rows 8 g + 4 kh + e, g, e = 0 ... 3 (register 4 g + e): dealt out so that these are
+    // the 16 consecutive columns of strip kh of the pair (two 16-byte accesses per output row), or, for the split-K form,
+    // whose blocks are not transposed, operand row = column (a store covers 128 consecutive bytes)
+    int const lane_slot = SPLITK ? row_in >> 4 : (row_in >> 2) & 1;
+    int const lane_col = SPLITK ? row_in & 15 : (row_in >> 3) * 4 + (row_in & 3);
     auto make_ctx = [&](int tm_, int tn_, bool valid) -> TileCtx
     {
         TileCtx x;
         int const first = tn_ * (kGemmBN / 16) + wave * NS;
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
+        for (int cb = 0; cb < CB; ++cb)
         {
-            int const strip = first + s < p.strips ? first + s : p.strips - 1;
-            x.wlane[s] = ((uint32_t) strip * (uint32_t) p.k_tiles * 64u + (uint32_t) lane) * 16u;
-            x.sc_lane[s] = (uint32_t) (strip * 16 + c) * 2u;
+            int const want = first + 2 * cb + lane_slot, strip = want < p.strips ? want : p.strips - 1;
+            x.wlane[cb] = ((uint32_t) strip * (uint32_t) p.k_tiles * 64u + (uint32_t) (kh * 32 + lane_col)) * 16u;
+            x.sc_lane[cb] = (uint32_t) (strip * 16 + lane_col) * 2u;
         }
         // A tile -> LDS: wavefront w moves pairs w, w+4, ...: piece i is pair f = w + 4i = half w % 2 of
         // row tile 2i + w / 2
@@ -119,356 +140,340 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     };
     TileCtx cur = make_ctx(tm, tn, true);
 
-    f32x4 acc[RT][NS];
+    f32x16 acc[RB][CB];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
-            acc[rt][s] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int cb = 0; cb < CB; ++cb)
+            acc[rb][cb] = f32x16{};
 
     // ---- A tile -> LDS; K is a multiple of 128, so only kt >= KT falls out of range (rows past M fall
     // outside the descriptor by themselves).
-    constexpr int DMA_OPS = PAIRS / 4;
-    uint32_t const dma_piece_stride = 32u * (uint32_t) K;
+    constexpr int DMA_OPS = PAIRS / NW;
+    uint32_t const dma_piece_stride = (uint32_t) NW * 8u * (uint32_t) K;
     auto dma_base = [&](int kt, TileCtx const& x) -> uint32_t
     { return (x.dma_lane_base + (uint32_t) kt * (uint32_t) TK) | ((uint32_t) (KT - 1 - kt) & kOob) | x.oob; };
     auto dma_piece = [&](auto* buf, uint32_t base, int i)
     {
-        int const f = wave + i * 4;
+        int const f = wave + i * NW;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(act_rsrc,
             (__attribute__((address_space(3))) void*) (reinterpret_cast<char*>(buf) + f * 1024), 16,
             (int) (base + (uint32_t) i * dma_piece_stride), 0, 0, 0);
     };
-    // MFMA lane (kg, c), slab j = 2*jp + jj of row tile rt: row c, bytes jj*32 + kg*8 .. +8 of the
-    // pair's 64: chunk jj*2 + kg/2 (stored at position chunk ^ (c>>2)), half kg & 1
+    // Matrix instruction ki of a tile row covers slabs 2 ki and 2 ki + 1; lane (kh, row_in) supplies the 16 values
+    // 32 j + 16 kh ... of each - two consecutive chunks of 8 of the weight layout, one 16-byte read of the activations:
+    // chunk (j & 1) * 2 + kh of row row_in % 16 in fragment pair ki, stored at position chunk ^ swizzle (the phases of a
+    // 128-bit LDS read take rows 0-3, 12-15 of one fragment and rows 4-11 of the other: all banks, no conflict)
     uint32_t a_lane_off[2];
 #pragma unroll
     for (int jj = 0; jj < 2; ++jj)
-        a_lane_off[jj] = (uint32_t) ((c * 4 + ((jj * 2 + (kg >> 1)) ^ ((c >> 2) & 3))) * 16 + (kg & 1) * 8);
+        a_lane_off[jj] = (uint32_t) ((row_in >> 4) * 2048 + ((row_in & 15) * 4 + ((jj * 2 + kh) ^ ((row_in >> 2) & 3))) * 16);
 
     struct BStage
     {
-        u32x4 w[NS];
-        uint16_t s[NS];
-        uint16_t z[NS];
+        u32x4 w[NS]; // [column block][chunk 2 kh, 2 kh + 1]
+        uint32_t s[CB]; // (32 bits: a 16-bit loop variable is merged into its register by an instruction that waits for the load)
+        uint32_t z[CB];
     };
-    constexpr int FETCH_OPS = NS * (ZERO ? 3 : 2);
+    constexpr int FETCH_OPS = NS + CB * (ZERO ? 2 : 1);
     auto fetch_piece = [&](BStage& st, int kt, int i, TileCtx const& x)
     {
         uint32_t const past = ((uint32_t) (KT - 1 - kt) & kOob) | x.oob; // kt >= KT: every load of the step reads zeros
         if (i < NS)
-            st.w[i] = buffer_load_x4(w_rsrc, x.wlane[i] + ((uint32_t) kt * 1024u | past));
+            st.w[i] = buffer_load_x4(w_rsrc, x.wlane[i / 2] + (((uint32_t) kt * 1024u | past) + (uint32_t) (i % 2 * 256)));
         else
         {
-            int const s = (i - NS) % NS;
-            uint32_t const off = (w4a8_scale_row((uint32_t) kt, magic) * (uint32_t) p.n * 2u + x.sc_lane[s]) | past;
-            if (i < 2 * NS)
+            int const s = (i - NS) % CB;
+            uint32_t const off = (__umulhi((uint32_t) kt * 2u, magic) * (uint32_t) p.n * 2u + x.sc_lane[s]) | past;
+            if (i < NS + CB)
                 st.s[s] = buffer_load_u16(sc_rsrc, off);
             else
                 st.z[s] = buffer_load_u16(zr_rsrc, off);
         }
     };
 
-    // ---- one step = one tile row of K = RT iterations of 4 MFMAs (one per strip).  Iteration rt
-    // issues the activation reads of the row tile A_AHEAD ahead, its share of the memory requests
-    // (packed weights of step kt+2, A tile of step kt+1) and of the conversions that build the B
-    // operands of step kt+1 (32 half-operands of 4 weights), then the 4 MFMAs of row tile rt.
+    // ---- one step = one tile row of K = KI * RB iterations of one MFMA.  Iteration (ki, rb)
+    // issues the activation reads of the operand A_AHEAD ahead, its share of the memory requests
+    // and of the conversions, then the MFMA of the row block.
+    // The operands of one instruction along K (8 registers) are all there is of converted weights: while the row blocks
+    // are multiplied with those of ki = 0, ki = 1 of the same step is converted, meanwhile ki = 0 of the next step.
+    // Conversion is a look-up (w4a8_common.h): a (group, column) has sixteen possible e4m3 results; the two lanes that feed
+    // a column each compute eight of them - the same FMA and saturating conversion as dequant2_fp8, so the bytes are
+    // identical, with zero-points or without - and exchange them.  15 instructions per eight weights against 21 issue slots
+    // of the arithmetic form (the conversion instruction takes two).
     constexpr int A_AHEAD = 2;
-    auto slab_at = [](int pos) { return ((pos & 1) << 1) | (pos >> 1); }; // its own inverse
-    // conversion unit cu = (strip, slab, half, pair): 2 weights -> 16 bits of the operand set.  The
-    // same arithmetic as dequant2_fp8 (w4a8_common.h), cut into four stages so that the main loop can
-    // run each stage of a unit behind a different matrix instruction: issued back to back, every
-    // instruction of the chain mask -> byte-to-float -> FMA -> pack waits for the one before it.
-    NibbleConsts const nib = nibble_consts<WOQ_FP16>(); // 0x000F000F in an SGPR, 0x64006400 (1024 as a pair of halves) in a VGPR
-    struct ConvState
+    Fp8LookupConsts const lut = fp8_lookup_consts();
+    f16x2 qv[4]; // the lane's eight signed values 8 kh - 8 ... 8 kh - 1, as halves for mixed-precision FMAs
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        qv[i] = f16x2{(_Float16) (8 * kh - 8 + 2 * i), (_Float16) (8 * kh - 7 + 2 * i)};
+    constexpr int TABLE_PARTS = 6; // of a table's construction: four pairs of entries, two exchanges
+    auto table_part = [&](Fp8Table& T, BStage const& st, int part)
     {
-        uint32_t src[2][2]; // zero-points: sign-flipped source word of (slab parity, pair)
-        uint32_t pw[16];    // no zero-points: the unit's two nibbles as a pair of halves 1024 + u (1024 + 16 u for pr = 1)
-        uint32_t sh;        // no zero-points: the slab word shifted by 8 (made by the unit h = 1, pr = 0 for both pairs)
-        float v[16][2];     // the two values of the units in flight (unit % 16: at most 12 are)
-    };
-    auto conv_stage = [&](ConvState& cs, u32x8 (&b)[NS], BStage const& st, int cu, int stage)
-    {
-        int const s = cu / 16, j = (cu / 4) % 4, h = (cu / 2) % 2, pr = cu % 2;
-        float(&v)[2] = cs.v[cu % 16];
-        if constexpr (ZERO)
+        if (part < 4)
         {
-            // fma(q, s, z) on the two's-complement nibble: q/16 straight from the nibble, times 16 s
-            uint32_t& src = cs.src[j & 1][pr];
-            if (stage == 0)
-            {
-                if (h != 0)
-                    return; // the unit with h = 0 made the word for both
-                uint32_t const w = st.w[s][j] ^ 0x88888888u; // biased -> two's complement nibbles
-                src = pr == 0 ? w : (w >> 4);
-                // (here and below: an anchor in the order of the volatile statements, i.e. of the matrix
-                // instructions - the next stage's instructions cannot be moved up to this one's)
-                asm volatile("" : "+v"(src));
-            }
-            else if (stage == 1)
-            {
-                v[0] = cvt_off_f32_i4_byte(src, h);
-                v[1] = cvt_off_f32_i4_byte(src, h + 2);
-                asm volatile("" : "+v"(v[0]), "+v"(v[1]));
-            }
-            else if (stage == 2)
-            {
-                float const sc = EH::from_bits(st.s[s]), zr = EH::from_bits(st.z[s]);
-                v[0] = __builtin_fmaf(v[0], 16.f * sc, zr);
-                v[1] = __builtin_fmaf(v[1], 16.f * sc, zr);
-                asm volatile("" : "+v"(v[0]), "+v"(v[1]));
-            }
+            _Float16 const sh = bit_cast<_Float16>((uint16_t) st.s[0]);
+            _Float16 const zh = bit_cast<_Float16>((uint16_t) (ZERO ? st.z[0] : 0u));
+            float const v0 = __builtin_fmaf((float) qv[part][0], (float) sh, (float) zh);
+            float const v1 = __builtin_fmaf((float) qv[part][1], (float) sh, (float) zh);
+            uint32_t& d = T.t[part / 2];
+            d = part % 2 == 0 ? (uint32_t) __builtin_amdgcn_cvt_pk_fp8_f32(v0, v1, 0, false)
+                              : (uint32_t) __builtin_amdgcn_cvt_pk_fp8_f32(v0, v1, (int) d, true);
         }
-        else
+        else // lanes below 32 have entries 0 ... 7, the others 8 ... 15
         {
-            // q s = fma(1024 + u, s, -1032 s) on the stored nibble u = q + 8: elements e0 = 4h + 2pr and
-            // e0 + 1 sit in nibbles e0/2 and e0/2 + 4, i.e. 16 bits apart - one and-or makes the pair
-            // of halves 0x6400 | u = 1024 + u, which the FMA reads directly.  The pair pr = 1 is taken
-            // where it sits, four bits up (still inside a half's ten fraction bits): 1024 + 16 u, and
-            // q s = fma(1024 + 16 u, s / 16, -72 s); so only the units of h = 1 need a shift, one for
-            // both.  The constants and the result (15 significant bits) are exact in float32: the same
-            // single rounding to e4m3 as fma(q, s, 0).
-            uint32_t& pw = cs.pw[cu % 16];
-            if (stage == 0)
-            {
-                if (h == 1 && pr == 0)
-                {
-                    cs.sh = st.w[s][j] >> 8;
-                    asm volatile("" : "+v"(cs.sh));
-                }
-                uint32_t const src = h == 0 ? st.w[s][j] : cs.sh;
-                pw = (src & (pr == 0 ? nib.mask : nib.mask << 4)) | nib.magic; // one v_and_or_b32
-                asm volatile("" : "+v"(pw));
-            }
-            else if (stage == 2)
-            {
-                float const sc = EH::from_bits(st.s[s]);
-                f16x2 const pair = bit_cast<f16x2>(pw);
-                float const mul = pr == 0 ? sc : 0.0625f * sc, add = pr == 0 ? -1032.f * sc : -72.f * sc;
-                v[0] = __builtin_fmaf((float) pair[0], mul, add);
-                v[1] = __builtin_fmaf((float) pair[1], mul, add);
-                asm volatile("" : "+v"(v[0]), "+v"(v[1]));
-            }
-        }
-        if (stage == 3)
-        {
-            int const idx = slab_at(j) * 2 + h; // slab j sits at operand position slab_at(j)
-            b[s][idx] = pr == 0 ? (uint32_t) __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], (int) b[s][idx], false)
-                                : (uint32_t) __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], (int) b[s][idx], true);
+            uint32_t const own = T.t[part - 4];
+            auto const both = __builtin_amdgcn_permlane32_swap(own, own, false, false);
+            T.t[part - 4] = both[0];
+            T.t[part - 2] = both[1];
         }
     };
-    // all four stages of one unit at once (prologue)
-    auto convert_unit = [&](u32x8 (&b)[NS], BStage const& st, int cu)
+    // look-up unit u = (slab parity, load) of instruction ki: eight weights -> two registers of its operand
+    constexpr int UNITS = 4;
+    auto unit_word = [&](BStage const& st, int ki, int u) { return st.w[u & 1][2 * ki + (u >> 1)]; };
+    auto unit_begin = [&](uint32_t (&part)[4], Fp8Table const& T, BStage const& st, int ki, int u)
+    { fp8_lookup8_begin(unit_word(st, ki, u), T, lut, part); };
+    auto unit_end = [&](uint32_t const (&part)[4], u32x8& b, BStage const& st, int ki, int u)
     {
-        int const s = cu / 16, j = (cu / 4) % 4, h = (cu / 2) % 2, pr = cu % 2;
-        int const idx = slab_at(j) * 2 + h;
-        float const sc = EH::from_bits(st.s[s]);
-        float const zr = ZERO ? EH::from_bits(st.z[s]) : 0.f;
-        b[s][idx] = dequant2_fp8<ZERO, false>(b[s][idx], st.w[s][j], h, pr, sc, zr);
+        uint32_t lo, hi;
+        fp8_lookup8_end(unit_word(st, ki, u), lut, part, lo, hi);
+        b[u * 2] = lo;
+        b[u * 2 + 1] = hi;
     };
-    constexpr int UNITS = NS * SLABS * 4; // 64 per step
 
-    // PERSIST: where the finished tile's outputs go: byte offset of (row m0 + c, column strip0 * 16 + kg * 4)
+    // PERSIST: where the finished tile's outputs go: byte offset of (row m0 + row_in, column strip0 * 16 + kh * 16)
     // of the tile to store (N is a multiple of the tile width: every strip exists; rows past M fall
     // outside the descriptor); kOob: no finished tile yet
     [[maybe_unused]] auto const out_rsrc = make_rsrc(p.out, (uint32_t) p.m * (uint32_t) p.n * 2u);
     [[maybe_unused]] uint32_t prev_off = kOob;
-    [[maybe_unused]] uint32_t const rt_stride = 16u * (uint32_t) p.n * 2u;
-    auto store_block = [&](int rt, int s)
+    [[maybe_unused]] uint32_t const rb_stride = (uint32_t) BLK * (uint32_t) p.n * 2u;
+    auto store_block = [&](int rb, int cb)
     {
         // explicit AGPR-source moves: a plain VALU use of the block would pull every accumulator into the
         // VGPR half of the file for the whole loop.  The pack to bf16 does not depend on the conversion
         // mode the main loop runs in (that concerns fp16 and fp8 results only).
-        float v[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[r]) : "a"(acc[rt][s][r]));
-        u32x2 const o = {EO::pack(p.alpha * v[0], p.alpha * v[1]), EO::pack(p.alpha * v[2], p.alpha * v[3])};
-        __builtin_amdgcn_raw_buffer_store_b64(o, out_rsrc, (int) (prev_off + (uint32_t) rt * rt_stride + (uint32_t) s * 32u), 0, 0);
-    };
-
-    // One step.  The A tile of step kt_a of tile xa goes to buf_next, the packed weights of step kt_w of
-    // tile xw to st_req (the steps after this one and after the next: the same tile's, or with PERSIST
-    // the next tile's first ones).  first_tag: the first step of a tile in the persistent loop.
-    auto compute = [&](auto first_tag, auto const* buf, u32x8 const (&b_use)[NS], u32x8 (&b_make)[NS],
-                       BStage const& st_conv, BStage& st_req, auto* buf_next, int kt_a, TileCtx const& xa, int kt_w,
-                       TileCtx const& xw)
-    {
-        constexpr bool FIRST = decltype(first_tag)::value;
-        char const* a_base = reinterpret_cast<char const*>(buf);
-        uint32_t const next_base = dma_base(kt_a, xa);
-        auto a_read = [&](int rt) -> u32x8
+        for (int h = 0; h < 2; ++h)
         {
-            // operand position pos holds slab slab_at(pos) = 0, 2, 1, 3: the two pieces that sit
-            // 1 KiB apart in LDS (same half of the two fragment pairs) come from one two-address read
-            u32x8 a;
+            float v[8];
 #pragma unroll
-            for (int pos = 0; pos < SLABS; ++pos)
-            {
-                int const j = slab_at(pos);
-                u32x2 const v = *reinterpret_cast<u32x2 const*>(a_base + (rt * 2 + j / 2) * 1024 + a_lane_off[j % 2]);
-                a[2 * pos] = v[0];
-                a[2 * pos + 1] = v[1];
-            }
-            return a;
-        };
-        u32x8 a_ring[A_AHEAD + 1];
+            for (int x = 0; x < 8; ++x)
+                asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[x]) : "a"(acc[rb][cb][h * 8 + x]));
+            u32x4 o;
 #pragma unroll
-        for (int i = 0; i < A_AHEAD && i < RT; ++i)
-            a_ring[i] = a_read(i);
-        // the conversion pipeline's head: the stages that the first matrix instructions expect done
-        constexpr int PER0 = UNITS / (RT * NS);
-        ConvState cs;
-        constexpr bool PIPELINED = RT >= 8; // (64-row tiles measured 2-8 % faster without the stage pipeline, 128-row tiles 3-6 % slower)
-#pragma unroll
-        for (int lead = 0; PIPELINED && lead < 3; ++lead)
-#pragma unroll
-            for (int stage = 0; stage < 3 - lead; ++stage)
-#pragma unroll
-                for (int x = 0; x < PER0; ++x)
-                    if (lead * PER0 + x < UNITS)
-                        conv_stage(cs, b_make, st_conv, lead * PER0 + x, stage);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-        {
-            // the A-tile DMAs first, the weight-side requests of step kt+2 after them: the barrier
-            // that ends the step then waits for the DMAs only (vector-memory operations retire in
-            // order) and leaves the weight loads, which travel from HBM, a whole further step
-            constexpr int DMA_WINDOW = RT / 2 > 0 ? RT / 2 : 1;
-#pragma unroll
-            for (int q = 0; q < DMA_OPS; ++q)
-                if (q * DMA_WINDOW / DMA_OPS == rt)
-                    dma_piece(buf_next, next_base, q);
-            constexpr int FETCH_FIRST = RT / 2, FETCH_WINDOW = RT - RT / 2 - 1 > 0 ? RT - RT / 2 - 1 : 1;
-#pragma unroll
-            for (int q = 0; q < FETCH_OPS; ++q)
-                if (FETCH_FIRST + q * FETCH_WINDOW / FETCH_OPS == rt)
-                    fetch_piece(st_req, kt_w, q, xw);
-            if (rt + A_AHEAD < RT)
-                a_ring[(rt + A_AHEAD) % (A_AHEAD + 1)] = a_read(rt + A_AHEAD);
-            u32x8 const a_cur = a_ring[rt % (A_AHEAD + 1)];
-            // one MFMA, then its share of the conversions: a wavefront issues in order, so the
-            // VALU work has to sit between the matrix instructions to run under them
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-            {
-                // weights as the first operand: the accumulator holds the TRANSPOSED 16x16 block, lane
-                // (kg, c) the four consecutive columns kg*4 .. kg*4+3 of output row c (8-byte epilogue accesses)
-                // (the split-K variant keeps the plain orientation: its float32 stores cover 64 consecutive
-                // bytes per row and instruction)
-                if constexpr (SPLITK)
-                    mma_fp8_acc(a_cur, b_use[s], acc[rt][s]);
-                else if constexpr (FIRST)
-                {
-                    store_block(rt, s); // the previous tile's sums leave right before the block starts the new tile's
-                    mma_fp8_first(b_use[s], a_cur, acc[rt][s]);
-                }
-                else
-                    mma_fp8_acc(b_use[s], a_cur, acc[rt][s]);
-                // behind matrix instruction t: the pack of the units whose FMAs went behind t - 1, the
-                // FMAs of those converted behind t - 2, and so on (PER units per instruction)
-                constexpr int PER = UNITS / (RT * NS);
-                int const t = rt * NS + s;
-                if constexpr (PIPELINED)
-                {
-#pragma unroll
-                    for (int stage = 3; stage >= 0; --stage)
-#pragma unroll
-                        for (int x = 0; x < PER; ++x)
-                        {
-                            int const cu = (t + 3 - stage) * PER + x;
-                            if (cu < UNITS)
-                                conv_stage(cs, b_make, st_conv, cu, stage);
-                        }
-                }
-                else
-                {
-                    // fewer row tiles: several units per matrix instruction, independent of each other -
-                    // each goes through its four stages here
-#pragma unroll
-                    for (int x = 0; x < PER; ++x)
-#pragma unroll
-                        for (int stage = 0; stage < 4; ++stage)
-                            conv_stage(cs, b_make, st_conv, t * PER + x, stage);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            for (int x = 0; x < 8; x += 2)
+                o[x / 2] = EO::pack(p.alpha * v[x], p.alpha * v[x + 1]);
+            __builtin_amdgcn_raw_buffer_store_b128(
+                o, out_rsrc, (int) (prev_off + (uint32_t) rb * rb_stride + (uint32_t) (cb * 64 + h * 16)), 0, 0);
         }
     };
 
-    // ---- main loop: two steps per iteration so that LDS buffers, operand sets and weight stages
-    // are distinct objects.  Step kt multiplies with operand set kt%2 (converted during step kt-1
-    // from weight stage kt%2), converts set (kt+1)%2 from stage (kt+1)%2 and refills stage kt%2
-    // with the packed weights of step kt+2.  (Requesting the weights a further step ahead - four
-    // stages - measured the same.)
-    BStage st0, st1;
-    u32x8 b0[NS], b1[NS];
-    fp8_saturation_on(); // the conversions rely on it; off again before the epilogue
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-        b0[s] = b1[s] = u32x8{0, 0, 0, 0, 0, 0, 0, 0};
+    // One step.  buf / buf_after: the A tiles of this step and (DEEP) of the next one, both landed; the last iterations
+    // already read the next step's first operands.  The A tile of tile row kt_a of tile xa goes to buf_req, the packed
+    // weights of tile row kt_w of tile xw to st_req - three steps ahead (not DEEP: one and two): the same tile's, or with
+    // PERSIST the next tile's first ones.  first_tag: the first step of a tile in the persistent loop.
+    constexpr int ITERS = RB * KI;
+    constexpr int A_RING = 4; // slots; A_AHEAD + 1 are in use
+    static_assert(ITERS % A_RING == 0, "a step starts on slot 0");
+    u32x8 a_ring[A_RING];
+    auto a_read = [&](auto const* buf, int it) -> u32x8 // row block it % RB, instruction it / RB of a tile row
     {
-        uint32_t const base = dma_base(kt_begin, cur);
+        char const* const at = reinterpret_cast<char const*>(buf) + (it % RB) * 4096 + (it / RB) * 1024;
+        u32x4 const lo = *reinterpret_cast<u32x4 const*>(at + a_lane_off[0]);
+        u32x4 const hi = *reinterpret_cast<u32x4 const*>(at + a_lane_off[1]);
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    u32x8 b[KI]; // converted weights, by instruction along K
+    auto compute = [&](auto first_tag, auto const* buf, auto const* buf_after, Fp8Table const& T, Fp8Table& T_next,
+                       BStage const& st, BStage const& st_next, auto* buf_req, int kt_a, TileCtx const& xa, BStage& st_req,
+                       int kt_w, TileCtx const& xw) __attribute__((always_inline))
+    {
+        constexpr bool FIRST = decltype(first_tag)::value;
+        uint32_t const next_base = dma_base(kt_a, xa);
+        if constexpr (!DEEP)
+        {
+#pragma unroll
+            for (int i = 0; i < A_AHEAD; ++i)
+                a_ring[i] = a_read(buf, i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t part[4];
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it)
+        {
+            // the A-tile DMAs first, the weight-side requests after them: with kPersistPairs the barrier
+            // that ends the step then waits for the DMAs only (vector-memory operations retire in
+            // order) and leaves the weight loads, which travel from HBM, a whole further step
+            constexpr int DMA_WINDOW = ITERS / 2 > 0 ? ITERS / 2 : 1;
+#pragma unroll
+            for (int q = 0; q < DMA_OPS; ++q)
+                if (q * DMA_WINDOW / DMA_OPS == it)
+                    dma_piece(buf_req, next_base, q);
+            constexpr int FETCH_FIRST = ITERS / 2, FETCH_WINDOW = ITERS - ITERS / 2 - 1 > 0 ? ITERS - ITERS / 2 - 1 : 1;
+#pragma unroll
+            for (int q = 0; q < FETCH_OPS; ++q)
+                if (FETCH_FIRST + q * FETCH_WINDOW / FETCH_OPS == it)
+                    fetch_piece(st_req, kt_w, q, xw);
+            if (DEEP || it + A_AHEAD < ITERS)
+                a_ring[(it + A_AHEAD) % A_RING]
+                    = it + A_AHEAD < ITERS ? a_read(buf, it + A_AHEAD) : a_read(buf_after, it + A_AHEAD - ITERS);
+            u32x8 const a_cur = a_ring[it % A_RING];
+            int const rb = it % RB, ki = it / RB;
+            // weights as the first operand: the accumulator holds the TRANSPOSED block, a lane 16
+            // consecutive columns of one output row (16-byte epilogue accesses)
+            // (the split-K variant keeps the plain orientation: its float32 stores cover 128 consecutive
+            // bytes per row and instruction)
+            if constexpr (SPLITK)
+                mma_fp8_acc<RT == 16>(a_cur, b[ki], acc[rb][0]);
+            else if (FIRST && ki == 0)
+            {
+                store_block(rb, 0); // the previous tile's sums leave right before the block starts the new tile's
+                mma_fp8_first<RT == 16>(b[ki], a_cur, acc[rb][0]);
+            }
+            else
+                mma_fp8_acc<RT == 16>(b[ki], a_cur, acc[rb][0]);
+            // behind the MFMA its share of the conversions, half units at a time: a wavefront issues in order, so the
+            // VALU work has to sit between the matrix instructions to run under them
+            BStage const& src = ki == 0 ? st : st_next;
+            Fp8Table const& table = ki == 0 ? T : T_next;
+#pragma unroll
+            for (int half = 0; half < 2 * UNITS; ++half)
+                if (half * RB / (2 * UNITS) == rb)
+                {
+                    if (half % 2 == 0)
+                        unit_begin(part, table, src, 1 - ki, half / 2);
+                    else
+                        unit_end(part, b[1 - ki], src, 1 - ki, half / 2);
+                }
+            if (ki == 0)
+            {
+#pragma unroll
+                for (int i = 0; i < TABLE_PARTS; ++i)
+                    if (i * RB / TABLE_PARTS == rb)
+                        table_part(T_next, st_next, i);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    // ---- main loop: four steps per iteration so that LDS buffers and weight stages
+    // are distinct objects.  Step kt converts ki = 1 of its own weights (stage kt % 4) and ki = 0 of the next step's and
+    // requests A tile and weights of step kt+3.  (kPersistPairs: two steps per iteration, two buffers and stages; A tile
+    // of step kt+1, weights of step kt+2.)
+    BStage st0, st1, st2, st3;
+    Fp8Table t0, t1;
+    fp8_saturation_on(); // the conversions rely on it; off again before the epilogue
+    auto request_a = [&](auto* buf, int kt)
+    {
+        uint32_t const base = dma_base(kt, cur);
 #pragma unroll
         for (int i = 0; i < DMA_OPS; ++i)
-            dma_piece(a_buf0, base, i);
+            dma_piece(buf, base, i);
+    };
+    auto request_w = [&](BStage& st, int kt)
+    {
+#pragma unroll
+        for (int i = 0; i < FETCH_OPS; ++i)
+            fetch_piece(st, kt, i, cur);
+    };
+    request_a(a_buf0, kt_begin);
+    request_w(st0, kt_begin);
+    if constexpr (DEEP)
+        request_a(a_buf1, kt_begin + 1);
+    request_w(st1, kt_begin + 1);
+    if constexpr (DEEP)
+    {
+        request_a(a_buf2, kt_begin + 2);
+        request_w(st2, kt_begin + 2);
     }
 #pragma unroll
-    for (int i = 0; i < FETCH_OPS; ++i)
-        fetch_piece(st0, kt_begin, i, cur);
+    for (int i = 0; i < TABLE_PARTS; ++i)
+        table_part(t0, st0, i);
 #pragma unroll
-    for (int i = 0; i < FETCH_OPS; ++i)
-        fetch_piece(st1, kt_begin + 1, i, cur);
-#pragma unroll
-    for (int cu = 0; cu < UNITS; ++cu)
-        convert_unit(b0, st0, cu);
-    // A(kt) has landed for every wavefront (at most the FETCH_OPS weight-side loads issued after its
-    // DMAs are still outstanding: loads return in order, and the persistent loop's stores are older than
-    // the last of them too); everyone is done reading the other buffer
-    auto step_barrier = [&]() { asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(FETCH_OPS) : "memory"); };
+    for (int u = 0; u < UNITS; ++u)
+    {
+        uint32_t part[4];
+        unit_begin(part, t0, st0, 0, u);
+        unit_end(part, b[0], st0, 0, u);
+    }
+    // DEEP: A(kt) and A(kt+1) have landed for every wavefront (the requests of the step before, DMA_OPS + FETCH_OPS loads,
+    // may still be out: loads return in order, whatever stores the persistent loop has issued between them); everyone is
+    // done reading A(kt-1), whose buffer this step's requests go to.  Else: A(kt) has landed (FETCH_OPS weight-side
+    // loads were requested after it).
+    auto step_barrier = [&]()
+    { asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(DEEP ? DMA_OPS + FETCH_OPS : FETCH_OPS) : "memory"); };
     std::false_type const plain{};
+    auto deep_step = [&](auto tag, auto const* buf, auto const* buf_after, Fp8Table const& T, Fp8Table& T_next, BStage const& st,
+                         BStage const& st_next, auto* buf_req, BStage& st_req, int kt, TileCtx const& x) __attribute__((always_inline))
+    {
+        compute(tag, buf, buf_after, T, T_next, st, st_next, buf_req, kt, x, st_req, kt, x);
+        step_barrier();
+    };
+    // tile rows kt ... kt+3 (past the end of K both operands read as zeros); the last three requests may be another tile's
+    auto four_steps = [&](auto tag, int kt, TileCtx const& x, int kt_x) __attribute__((always_inline))
+    {
+        deep_step(tag, a_buf0, a_buf1, t0, t1, st0, st1, a_buf3, st3, kt + 3, cur);
+        deep_step(plain, a_buf1, a_buf2, t1, t0, st1, st2, a_buf0, st0, kt_x, x);
+        deep_step(plain, a_buf2, a_buf3, t0, t1, st2, st3, a_buf1, st1, kt_x + 1, x);
+        compute(plain, a_buf3, a_buf0, t1, t0, st3, st0, a_buf2, kt_x + 2, x, st2, kt_x + 2, x);
+        mma_settle(); // the compiler may move accumulators behind the loop and does not see that they are still being written
+        step_barrier();
+    };
+    if constexpr (DEEP)
+    {
+        step_barrier();
+#pragma unroll
+        for (int i = 0; i < A_AHEAD; ++i)
+            a_ring[i] = a_read(a_buf0, i);
+    }
     if constexpr (!PERSIST)
     {
-        for (int kt = kt_begin; kt < KT; kt += 2)
+        int kt = kt_begin;
+        for (; kt + 2 < KT; kt += 4)
+            four_steps(plain, kt, cur, kt + 4);
+        if (kt < KT) // one or two left (leaving the loop from its middle would cost a second copy of the accumulators)
         {
-            step_barrier();
-            compute(plain, a_buf0, b0, b1, st1, st0, a_buf1, kt + 1, cur, kt + 2, cur);
-            step_barrier();
-            compute(plain, a_buf1, b1, b0, st0, st1, a_buf0, kt + 2, cur, kt + 3, cur); // past the end of K both operands read as zeros
+            deep_step(plain, a_buf0, a_buf1, t0, t1, st0, st1, a_buf3, st3, kt + 3, cur);
+            compute(plain, a_buf1, a_buf2, t1, t0, st1, st2, a_buf0, kt + 4, cur, st0, kt + 4, cur);
         }
     }
     else
     {
-        // Straight-line first, second and last two steps around a plain inner loop (KT even, >= 4; the
-        // shape the 16-bit kernel's persistent loop has, for the same reason: all 256 AGPRs are
-        // accumulators, and a branch between first-step and ordinary code inside a loop makes the
-        // allocator keep second copies of them).  Step kt multiplies operand set kt % 2 (buffer kt % 2),
-        // converts the weights of step kt + 1 and requests those of step kt + 2 and the A tile of step
-        // kt + 1 - in a tile's last two steps those are the next tile's first ones.
+        // Straight-line first and last steps around a plain inner loop (KT a multiple of 4, >= 8; in pairs: even, >= 4; the
+        // shape the 16-bit kernel's persistent loop has, for the same reason: every AGPR is an
+        // accumulator, and a branch between first-step and ordinary code inside a loop makes the
+        // allocator keep second copies of them).  In a tile's last three (two) steps the requests are the next tile's
+        // first ones.
         bool has_next;
         do
         {
             int tmn = 0, tnn = 0;
             has_next = tile_of(vb + (int) gridDim.x, tmn, tnn);
             TileCtx const nxt = make_ctx(tmn, tnn, has_next);
-            step_barrier();
-            compute(std::true_type{}, a_buf0, b0, b1, st1, st0, a_buf1, 1, cur, 2, cur);
-            step_barrier();
-            compute(plain, a_buf1, b1, b0, st0, st1, a_buf0, 2, cur, 3, cur);
-            for (int kt = 2; kt < KT - 2; kt += 2)
+            if constexpr (DEEP)
             {
-                step_barrier();
-                compute(plain, a_buf0, b0, b1, st1, st0, a_buf1, kt + 1, cur, kt + 2, cur);
-                step_barrier();
-                compute(plain, a_buf1, b1, b0, st0, st1, a_buf0, kt + 2, cur, kt + 3, cur);
+                four_steps(std::true_type{}, 0, cur, 4);
+                for (int kt = 4; kt < KT - 4; kt += 4)
+                    four_steps(plain, kt, cur, kt + 4);
+                four_steps(plain, KT - 4, nxt, 0);
             }
-            step_barrier();
-            compute(plain, a_buf0, b0, b1, st1, st0, a_buf1, KT - 1, cur, 0, nxt);
-            step_barrier();
-            compute(plain, a_buf1, b1, b0, st0, st1, a_buf0, 0, nxt, 1, nxt);
+            else
+            {
+                auto pair = [&](auto tag, int kt, TileCtx const& x, int kt_x) __attribute__((always_inline))
+                {
+                    step_barrier();
+                    compute(tag, a_buf0, a_buf0, t0, t1, st0, st1, a_buf1, kt + 1, cur, st0, kt_x, x);
+                    step_barrier();
+                    compute(plain, a_buf1, a_buf1, t1, t0, st1, st0, a_buf0, kt_x, x, st1, kt_x + 1, x);
+                    mma_settle();
+                };
+                pair(std::true_type{}, 0, cur, 2);
+                for (int kt = 2; kt < KT - 2; kt += 2)
+                    pair(plain, kt, cur, kt + 2);
+                pair(plain, KT - 2, nxt, 0);
+            }
             // this tile's outputs: stored during the next tile's first step (or below)
-            prev_off = ((uint32_t) (m0 + c) * (uint32_t) p.n + (uint32_t) (strip0 * 16 + kg * 4)) * 2u;
+            prev_off = ((uint32_t) (m0 + row_in) * (uint32_t) p.n + (uint32_t) (strip0 * 16 + kh * 16)) * 2u;
             vb += (int) gridDim.x;
             m0 = tmn * BM;
             strip0 = tnn * (kGemmBN / 16) + wave * NS;
@@ -477,10 +482,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         mma_drain();
         fp8_saturation_off();
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-            for (int s = 0; s < NS; ++s)
-                store_block(rt, s);
+            for (int cb = 0; cb < CB; ++cb)
+                store_block(rb, cb);
         return;
     }
 
@@ -489,51 +494,58 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     fp8_saturation_off();
     if constexpr (SPLITK)
     {
-        // plain orientation: acc[rt][s][r] = (row m0 + rt*16 + kg*4 + r, column strip*16 + c);
+        // plain orientation: register 4 g + e is (row rb * 32 + 8 g + 4 kh + e, the lane's own column);
         // this K slice's own slab of the partial buffer (a slice past the end of K stores zeros)
         float* const slab = p.partial + (size_t) blockIdx.y * ((size_t) p.m * p.n);
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
+        for (int cb = 0; cb < CB; ++cb)
+        {
+            int const strip = strip0 + 2 * cb + lane_slot;
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
+            for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
+                for (int r = 0; r < 16; ++r)
                 {
-                    int const row = m0 + rt * 16 + kg * 4 + r;
-                    if (strip0 + s < p.strips && row < p.m)
-                        slab[(size_t) row * p.n + (strip0 + s) * 16 + c] = acc[rt][s][r];
+                    int const row = m0 + rb * BLK + (r >> 2) * 8 + kh * 4 + (r & 3);
+                    if (strip < p.strips && row < p.m)
+                        slab[(size_t) row * p.n + strip * 16 + lane_col] = acc[rb][cb][r];
                 }
+        }
         return;
     }
     uint16_t* out16 = static_cast<uint16_t*>(p.out);
-    // acc[rt][s][r] = output (row m0 + rt*16 + c, column strip*16 + kg*4 + r): four consecutive
-    // columns per lane, written as one 8-byte store
-    typedef __attribute__((address_space(1))) u32x2 global_u32x2;
+    // a lane holds 16 consecutive columns of output row m0 + rb * 32 + row_in: two 16-byte stores
+    typedef __attribute__((address_space(1))) u32x4 global_u32x4;
 #pragma unroll
-    for (int s = 0; s < NS; ++s)
+    for (int cb = 0; cb < CB; ++cb)
     {
-        if (strip0 + s >= p.strips)
+        int const strip = strip0 + 2 * cb + kh;
+        if (strip >= p.strips)
             continue;
-        int const col = (strip0 + s) * 16 + kg * 4;
-        float bias[4] = {0.f, 0.f, 0.f, 0.f};
-        if (!SPLITK && p.bias)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
         {
+            int const col = strip * 16 + h * 8;
+            float bias[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (!SPLITK && p.bias)
+            {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                bias[r] = EO::load(p.bias, col + r);
-        }
+                for (int x = 0; x < 8; ++x)
+                    bias[x] = EO::load(p.bias, col + x);
+            }
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-        {
-            int const row = m0 + rt * 16 + c;
-            if (row >= p.m)
-                continue;
-            float v[4];
+            for (int rb = 0; rb < RB; ++rb)
+            {
+                int const row = m0 + rb * BLK + row_in;
+                if (row >= p.m)
+                    continue;
+                float v[8];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                v[r] = after_mode_change(__builtin_fmaf(p.alpha, acc[rt][s][r], bias[r]));
-            u32x2 const o = {EO::pack(v[0], v[1]), EO::pack(v[2], v[3])};
-            *(global_u32x2*) (out16 + (size_t) row * p.n + col) = o;
+                for (int x = 0; x < 8; ++x)
+                    v[x] = after_mode_change(__builtin_fmaf(p.alpha, acc[rb][cb][h * 8 + x], bias[x]));
+                u32x4 const o = {EO::pack(v[0], v[1]), EO::pack(v[2], v[3]), EO::pack(v[4], v[5]), EO::pack(v[6], v[7])};
+                *(global_u32x4*) (out16 + (size_t) row * p.n + col) = o;
+            }
         }
     }
 }
@@ -542,13 +554,13 @@ template <int ODT, bool ZERO, int RT>
 int launch_w4a8_variant(GemmParams const& gp, hipStream_t stream)
 {
     int const total = gp.tiles_m * gp.tiles_n;
-    dim3 grid(((total + 7) / 8) * 8, gp.k_splits), block(256);
+    dim3 grid(((total + 7) / 8) * 8, gp.k_splits), block(kW4a8Waves * 64);
     note_launch("gemm w4a8 rt=%d splits=%d", RT, gp.k_splits);
     if (gp.k_splits > 1)
     {
         size_t const count = (size_t) gp.m * gp.n;
         hipLaunchKernelGGL((gemm_w4a8_kernel<ODT, ZERO, RT, true>), grid, block, 0, stream, gp);
-        hipLaunchKernelGGL((gemm_finish_partial<ODT>), dim3((unsigned) ((count / 4 + 255) / 256)), block, 0, stream,
+        hipLaunchKernelGGL((gemm_finish_partial<ODT>), dim3((unsigned) ((count / 4 + 255) / 256)), dim3(256), 0, stream,
             gp.out, gp.partial, gp.bias, gp.alpha, gp.m, gp.n, gp.k_splits);
     }
     else
@@ -565,7 +577,12 @@ int launch_w4a8_variant(GemmParams const& gp, hipStream_t stream)
         if (persist)
         {
             if constexpr (RT == 16 && ODT == WOQ_BF16)
-                hipLaunchKernelGGL((gemm_w4a8_kernel<ODT, ZERO, RT, false, true>), dim3(cus), block, 0, stream, gp);
+            {
+                if (gp.k_tiles % 4 == 0 && gp.k_tiles >= 8)
+                    hipLaunchKernelGGL((gemm_w4a8_kernel<ODT, ZERO, RT, false, kPersist>), dim3(cus), block, 0, stream, gp);
+                else
+                    hipLaunchKernelGGL((gemm_w4a8_kernel<ODT, ZERO, RT, false, kPersistPairs>), dim3(cus), block, 0, stream, gp);
+            }
         }
         else
             hipLaunchKernelGGL((gemm_w4a8_kernel<ODT, ZERO, RT, false>), grid, block, 0, stream, gp);

@@ -162,6 +162,25 @@ __device__ __forceinline__ void fp8_lookup8(uint32_t w, Fp8Table const& T, Fp8Lo
     b1 = __builtin_amdgcn_perm(hi_o, lo_o, pick_o);
 }
 
+// The same in two parts, delivering the weights in their own order - bytes [e0 .. e3] and [e4 .. e7], two instructions
+// more - for kernels whose A operand comes straight out of LDS.
+__device__ __forceinline__ void fp8_lookup8_begin(uint32_t w, Fp8Table const& T, Fp8LookupConsts const& k, uint32_t (&part)[4])
+{
+    uint32_t const sel_e = w & k.low3, sel_o = (w >> 4) & k.low3;
+    part[0] = __builtin_amdgcn_perm(T.t[1], T.t[0], sel_e);
+    part[1] = __builtin_amdgcn_perm(T.t[3], T.t[2], sel_e);
+    part[2] = __builtin_amdgcn_perm(T.t[1], T.t[0], sel_o);
+    part[3] = __builtin_amdgcn_perm(T.t[3], T.t[2], sel_o);
+}
+
+__device__ __forceinline__ void fp8_lookup8_end(uint32_t w, Fp8LookupConsts const& k, uint32_t const (&part)[4], uint32_t& b0, uint32_t& b1)
+{
+    uint32_t const e = __builtin_amdgcn_perm(part[1], part[0], ((w >> 1) & k.bit2) | k.bytes); // [e0, e4, e1, e5]
+    uint32_t const o = __builtin_amdgcn_perm(part[3], part[2], ((w >> 5) & k.bit2) | k.bytes); // [e2, e6, e3, e7]
+    b0 = __builtin_amdgcn_perm(o, e, 0x06040200u);
+    b1 = __builtin_amdgcn_perm(o, e, 0x07050301u);
+}
+
 // eight consecutive k-values (bytes a0 .. a7 in v0, v1) in the order fp8_lookup8 delivers the weights
 __device__ __forceinline__ void fp8_a_order(uint32_t v0, uint32_t v1, uint32_t& a0, uint32_t& a1)
 {
@@ -237,6 +256,26 @@ __device__ __forceinline__ void mma_fp8_acc(u32x8 a, u32x8 b, f32x4& c)
 __device__ __forceinline__ void mma_fp8_first(u32x8 a, u32x8 b, f32x4& c)
 {
     asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
+}
+
+// the same on blocks of 32 x 32 x 64: twice the work for one issue slot.  AGPR: accumulators in the upper half of the
+// register file; the old value is an operand of the first product too, so that both name the same registers
+template <bool AGPR>
+__device__ __forceinline__ void mma_fp8_acc(u32x8 a, u32x8 b, f32x16& c)
+{
+    if constexpr (AGPR)
+        asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    else
+        asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+
+template <bool AGPR>
+__device__ __forceinline__ void mma_fp8_first(u32x8 a, u32x8 b, f32x16& c)
+{
+    if constexpr (AGPR)
+        asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
+    else
+        asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, 0" : "+v"(c) : "v"(a), "v"(b));
 }
 
 } // namespace woq
