@@ -639,7 +639,7 @@ EnvOverrides read_env()
     if (char const* e = std::getenv("WOQ_GEMM_RT"))
     {
         int const v = std::atoi(e);
-        o.gemm_rt = (v == 4 || v == 8 || v == 10 || v == 12 || v == 16) ? v : 0;
+        o.gemm_rt = (v == 1 || v == 4 || v == 8 || v == 10 || v == 12 || v == 16) ? v : 0;
     }
     if (char const* e = std::getenv("WOQ_GEMM_SPLITS"))
         o.gemm_splits = std::atoi(e);

@@ -34,6 +34,7 @@ struct GemmParams
     // and writes [m, n/2]; the strips of a wavefront then alternate between the two halves of N
     // (see paired_strip).  Other activations are applied by a separate pass.
     int activation = kActIdentity;
+    bool flex = false;   // grouped: row tiles of up to 128 rows, as tall as each expert needs (gemm_flex_kernel)
     int tile_cols = 256; // columns of an output tile of the exact-dequantize kernel (256, or 192 for 256-row tiles)
     void const* residual = nullptr; // [m, n_out] in the output type, added last (no split-K with it)
 };
@@ -81,6 +82,19 @@ inline void set_group_fields(GemmParams& gp, MatmulProblem const& p, int tile_ro
     gp.scale_stride = p.scale_stride;
     if (p.expert_rows) // every expert may end with a partly filled tile
         gp.tiles_m = p.m / tile_rows + p.num_experts;
+}
+
+// Grouped problems: row tiles of all experts together that have rows (the host launches an upper bound of them).  The lanes
+// of a wavefront take an expert each; the result is wavefront-uniform.
+__device__ __forceinline__ int count_expert_tiles(GemmParams const& p, int tile_rows)
+{
+    int tiles = 0;
+    for (int e = (int) (threadIdx.x & 63); e < p.num_experts; e += 64)
+        tiles += ((int) (p.expert_rows[e] - (e ? p.expert_rows[e - 1] : 0)) + tile_rows - 1) / tile_rows;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1)
+        tiles += __shfl_xor(tiles, d);
+    return __builtin_amdgcn_readfirstlane(tiles);
 }
 
 // Grouped problems: row tile `tm` counts through the row tiles of expert 0, 1, ... in turn.

@@ -28,6 +28,7 @@
 namespace woq
 {
 
+constexpr int kFlexRt = 8;     // tallest tile of the grouped kernel that picks its heights itself
 constexpr int kGemmGroupM = 4; // m-tiles walked together so that concurrent workgroups share panels in L2
 
 // amdgpu_waves_per_eu: from ten row tiles on one wavefront per SIMD is the design point (up to 256 accumulator
@@ -49,8 +50,30 @@ constexpr int kGemmGroupM = 4; // m-tiles walked together so that concurrent wor
 //        reuse): neither the first-load latency of a tile nor its burst of 128 KiB of stores is
 //        paid with the matrix core idle.  Plain epilogue only (bias; no activation, no residual);
 //        K must be an even number of tile rows; m * n * 2 < 2 GiB (outputs go through a descriptor).
-template <int DT, int BITS, int GROUP, bool ZERO, int RT, bool SPLITK, bool PERSIST = false, int NS_ = 4>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 8 ? 2 : 1, RT <= 8 ? 2 : 1))) gemm_kernel(GemmParams p)
+template <int BITS, int RT>
+constexpr int kGemmBufVecs = RT * 16 * (BITS == 4 ? 128 : 64) * 2 / 16; // 16-byte vectors of one activation tile in LDS
+
+// Output tile of virtual block vb (the block index itself, or with PERSIST the block index plus a multiple of
+// the grid size, which is a multiple of 8 - a workgroup stays on its XCD's chunk of the order): XCD-contiguous chunks,
+// m fastest inside groups of kGemmGroupM.
+__device__ __forceinline__ bool gemm_tile_of(GemmParams const& p, int vb, int& tm, int& tn)
+{
+    int const total = p.tiles_m * p.tiles_n;
+    int const per_xcd = (total + 7) / 8;
+    int const t = (vb & 7) * per_xcd + (vb >> 3);
+    if ((vb >> 3) >= per_xcd || t >= total)
+        return false;
+    int const in_group = kGemmGroupM * p.tiles_n;
+    int const first_m = (t / in_group) * kGemmGroupM;
+    int const gsz = p.tiles_m - first_m < kGemmGroupM ? p.tiles_m - first_m : kGemmGroupM;
+    tm = first_m + (t % in_group) % gsz;
+    tn = (t % in_group) / gsz;
+    return true;
+}
+
+// One output tile (PERSIST: the tiles of a workgroup, from virtual block vb on) of a problem that is no longer grouped.
+template <int DT, int BITS, int GROUP, bool ZERO, int RT, bool SPLITK, bool PERSIST, int NS_>
+__device__ __forceinline__ void gemm_body(GemmParams const& p, u32x4* a_buf0, u32x4* a_buf1, int vb, int tm, int tn)
 {
     static_assert(!(PERSIST && SPLITK), "a persistent workgroup owns whole tiles");
     using E = Elem<DT>;
@@ -62,34 +85,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
     constexpr int SEG = segment_rows<GROUP, TK>(); // rows sharing one scale inside a tile row
     constexpr int SEGS = TK / SEG;
     constexpr int SEG_SLABS = SEG / 32;
-    constexpr int A_BYTES = kGemmBM * TK * 2;
-
-    __shared__ u32x4 a_buf0[A_BYTES / 16];
-    __shared__ u32x4 a_buf1[A_BYTES / 16];
-
-    // ---- which output tile: XCD-contiguous chunks, m fastest inside groups of kGemmGroupM ------
-    // (virtual block vb: the block index itself, or with PERSIST the block index plus a multiple of
-    // the grid size, which is a multiple of 8 - a workgroup stays on its XCD's chunk of the order)
-    int const total = p.tiles_m * p.tiles_n;
-    int const per_xcd = (total + 7) / 8;
-    auto tile_of = [&](int vb, int& tm_, int& tn_) -> bool
-    {
-        int const t = (vb & 7) * per_xcd + (vb >> 3);
-        if ((vb >> 3) >= per_xcd || t >= total)
-            return false;
-        int const in_group = kGemmGroupM * p.tiles_n;
-        int const first_m = (t / in_group) * kGemmGroupM;
-        int const gsz = p.tiles_m - first_m < kGemmGroupM ? p.tiles_m - first_m : kGemmGroupM;
-        tm_ = first_m + (t % in_group) % gsz;
-        tn_ = (t % in_group) / gsz;
-        return true;
-    };
-    int vb = (int) blockIdx.x;
-    int tm, tn;
-    if (!tile_of(vb, tm, tn))
-        return;
-    if (p.expert_rows && !select_expert(p, tm, kGemmBM))
-        return;
 
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -492,7 +487,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
                     // this tile's outputs: stored during the next tile's first tile row (or below)
                     prev_off = ((uint32_t) (m0 + c) * (uint32_t) p.n + (uint32_t) (strip0 * 16 + kg * 4)) * 2u;
                     vb += (int) gridDim.x;
-                    if (tile_of(vb, tm, tn))
+                    if (gemm_tile_of(p, vb, tm, tn))
                     {
                         m0 = tm * kGemmBM;
                         strip0 = tn * (BN / 16) + wave * NS;
@@ -677,10 +672,81 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
         plain_epilogue(std::false_type{});
 }
 
+template <int DT, int BITS, int GROUP, bool ZERO, int RT, bool SPLITK, bool PERSIST = false, int NS = 4>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 8 ? 2 : 1, RT <= 8 ? 2 : 1))) gemm_kernel(GemmParams p)
+{
+    __shared__ u32x4 a_buf0[kGemmBufVecs<BITS, RT>];
+    __shared__ u32x4 a_buf1[kGemmBufVecs<BITS, RT>];
+    int tm, tn;
+    if (p.expert_rows) // the tiles that have rows, dealt evenly to the XCDs (with the empty ones at the end of the order one or
+        p.tiles_m = count_expert_tiles(p, RT * 16); // two XCDs would have little or nothing to do)
+    if (!gemm_tile_of(p, (int) blockIdx.x, tm, tn))
+        return;
+    if (p.expert_rows && !select_expert(p, tm, RT * 16))
+        return;
+    gemm_body<DT, BITS, GROUP, ZERO, RT, SPLITK, PERSIST, NS>(p, a_buf0, a_buf1, (int) blockIdx.x, tm, tn);
+}
+
+// Grouped problems with up to about 128 rows per expert: tiles as tall as an expert's rows ask for.  The host knows the
+// rows of all experts together only, and a common height either multiplies padding (128-row tiles on experts of 75 rows) or
+// converts the weights once more per expert (two 64-row tiles).  Here the workgroup divides its expert's rows into as
+// few tiles of up to 128 rows as they fit, all of one height, and runs the loop of that height.  All heights share
+// the 128-row loop's registers and LDS: two workgroups a CU.
+// Measured (8 experts, top-2 of T tokens, us, common height -> by expert): 4096 x 28672 with SwiGLU, fp16 per-channel, 150 /
+// 300 / 600 / 1000 tokens 151 -> 122 / 203 -> 162 / 324 -> 283 / 459 -> 384; bf16 group 128 at 300 / 600 tokens 268 -> 193 /
+// 384 -> 330; int8 at 300 288 -> 224.  About half of that is the order of the tiles: with the launch's upper bound of row
+// tiles dealt to the XCDs, the empty ones at its end left one or two XCDs idle (without that the first came out at 231).
+// What bounds it: conversions and matrix instructions in series (0.735 + 0.117 h us per 128 rows of K and tile of h row
+// tiles, two workgroups a CU), and the tallest expert's tile where the launch is a single round.
+template <int DT, int BITS, int GROUP, bool ZERO>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm_flex_kernel(GemmParams p)
+{
+    __shared__ u32x4 a_buf0[kGemmBufVecs<BITS, kFlexRt>];
+    __shared__ u32x4 a_buf1[kGemmBufVecs<BITS, kFlexRt>];
+    int tm, tn;
+    p.tiles_m = count_expert_tiles(p, kFlexRt * 16);
+    if (!gemm_tile_of(p, (int) blockIdx.x, tm, tn))
+        return;
+    if (!select_expert(p, tm, kFlexRt * 16))
+        return;
+    int const tiles = (p.m + kFlexRt * 16 - 1) / (kFlexRt * 16); // of this expert
+    // row tiles each needs to have (told to be uniform: the division runs on the vector unit)
+    int const height = __builtin_amdgcn_readfirstlane((p.m + tiles * 16 - 1) / (tiles * 16));
+    auto run = [&](auto rt_tag) __attribute__((always_inline))
+    {
+        constexpr int RT = decltype(rt_tag)::value;
+        gemm_body<DT, BITS, GROUP, ZERO, RT, false, false, 4>(p, a_buf0, a_buf1, 0, tm, tn);
+    };
+    // (int8: an even number of row tiles, whose activation fragments divide evenly over the wavefronts)
+    if (height <= 2)
+        run(std::integral_constant<int, 2>{});
+    else if (height <= 4)
+        run(std::integral_constant<int, 4>{});
+    else if (BITS == 4 && height == 5)
+        run(std::integral_constant<int, BITS == 4 ? 5 : 6>{});
+    else if (height <= 6)
+        run(std::integral_constant<int, 6>{});
+    else if (BITS == 4 && height == 7)
+        run(std::integral_constant<int, BITS == 4 ? 7 : 8>{});
+    else
+        run(std::integral_constant<int, 8>{});
+}
+
 template <int DT, int BITS, int GROUP, bool ZERO, int RT, int NS = 4>
 int launch_gemm_variant(GemmParams const& gp, hipStream_t stream)
 {
     static_assert(NS == 4 || RT == 16, "192-column tiles exist for the 256-row kernel only");
+    if constexpr (RT <= kFlexRt)
+    {
+        if (gp.flex)
+        {
+            note_launch("gemm exact rt=%d splits=1 persistent=0 columns=%d heights by expert", RT, NS * 64);
+            hipLaunchKernelGGL((gemm_flex_kernel<DT, BITS, GROUP, ZERO>), dim3(((gp.tiles_m * gp.tiles_n + 7) / 8) * 8), dim3(256), 0,
+                stream, gp);
+            hipError_t const e = hipGetLastError();
+            return e == hipSuccess ? WOQ_OK : fail(WOQ_ERR_RUNTIME, "gemm kernel launch failed: %s", hipGetErrorString(e));
+        }
+    }
     int const total = gp.tiles_m * gp.tiles_n;
     dim3 grid(((total + 7) / 8) * 8, gp.k_splits), block(256);
     if (gp.k_splits > 1)
@@ -771,7 +837,8 @@ int launch_gemm_typed(MatmulProblem const& p, GemmPlan const& plan, void* stream
     gp.partial = static_cast<float*>(p.workspace);
     if (plan.k_splits > 1 && (!p.workspace || p.workspace_bytes < plan.ws_bytes))
         return fail(WOQ_ERR_WORKSPACE, "split-K needs %zu workspace bytes", plan.ws_bytes);
-    set_group_fields(gp, p, plan.rt * 16);
+    gp.flex = plan.flex && p.expert_rows;
+    set_group_fields(gp, p, gp.flex ? kFlexRt * 16 : plan.rt * 16);
     auto s = static_cast<hipStream_t>(stream);
     bool const zero = p.zeros != nullptr;
     switch (template_group(p.group_size))

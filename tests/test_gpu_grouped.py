@@ -86,6 +86,35 @@ def test_grouped_160_and_192_row_tiles(pkg, oracle, dev, woq_env, rt, bits, grou
     assert oracle.max_rel_err(out, reference(oracle, p, "swiglu", residual)) < TOL
 
 
+@pytest.mark.parametrize("bits,group,zero,dtype", [(4, 128, True, "bf16"), (4, 0, False, "fp16"), (4, 64, False, "bf16"),
+                                                   (8, 0, False, "bf16"), (8, 128, True, "fp16")])
+@pytest.mark.parametrize("rows", [[16, 17, 32, 33, 48, 64, 65, 80], [81, 96, 97, 112, 113, 128, 129, 0], [300, 0, 1, 255, 257]])
+def test_grouped_heights_by_expert(pkg, oracle, dev, woq_env, rows, bits, group, zero, dtype):
+    """Every tile height of the kernel that picks them by expert (one row short of, at and past each), several tiles an
+    expert, empty experts, K of an odd number of tile rows, gated epilogue and residual: the oracle's bar, and the bits of
+    the fixed 128-row tiles (an output's sum runs over K in the same order whatever the height)."""
+    k = 320 if group == 64 else 384
+    p = grouped_problem(oracle, rows, k, 544, bits, group, dtype, zero, True, seed=sum(rows) + bits)
+    residual = oracle.round_to(np.random.default_rng(1).standard_normal((p["act"].shape[0], 272)).astype(np.float32), dtype)
+    woq_env(WOQ_GEMM_KERNEL="exact", WOQ_GEMM_RT="1")
+    out = run_grouped(pkg, oracle, dev, p, GEMM, "swiglu", residual=residual)
+    assert "heights by expert" in pkg._lib.lib.woq_last_launch().decode()
+    assert np.isfinite(out).all()
+    assert oracle.max_rel_err(out, reference(oracle, p, "swiglu", residual)) < TOL
+    woq_env(WOQ_GEMM_KERNEL="exact", WOQ_GEMM_RT="8")
+    assert np.array_equal(out, run_grouped(pkg, oracle, dev, p, GEMM, "swiglu", residual=residual))
+
+
+def test_grouped_more_experts_than_lanes(pkg, oracle, dev, woq_env):
+    """The tiles of 70 experts are counted by 64 lanes."""
+    rows = [(5 * e) % 23 for e in range(69)] + [130]
+    p = grouped_problem(oracle, rows, 128, 272, 4, 128, "bf16", True, False, seed=3)
+    woq_env(WOQ_GEMM_KERNEL="exact", WOQ_GEMM_RT="1")
+    out = run_grouped(pkg, oracle, dev, p, GEMM)
+    assert np.isfinite(out).all()
+    assert oracle.max_rel_err(out, reference(oracle, p)) < TOL
+
+
 def test_grouped_prefill_sizes(pkg, oracle, dev):
     """Hundreds of rows per expert: the exact-dequantize kernel with 256-row (or 128-row) tiles."""
     p = grouped_problem(oracle, [600, 300, 0, 700], 512, 512, 4, 128, "bf16", True, True, seed=9)
