@@ -15,7 +15,7 @@
 namespace woq
 {
 
-template <int DT, bool TO_FP8, int CHUNKS>
+template <int DT, bool TO_FP8, int CHUNKS, bool AHEAD>
 __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void const* x, void const* gamma,
     void const* beta, void const* scale, float eps, int k)
 {
@@ -24,13 +24,27 @@ __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void c
     uint16_t const* src = static_cast<uint16_t const*>(x) + row * k;
     int const n8 = k / 8; // 16-byte pieces of a row; thread t owns pieces t, t + 256, ...
 
-    u32x4 v[CHUNKS];
-    float ss = 0.f;
+    // AHEAD: the tables' pieces are requested together with the row's; read behind the sum of squares they cost a second
+    // trip to memory (us, bf16 -> e4m3 with smoothing: 8 x 8192 3.80 -> 3.46, 1990 x 4096 7.64 -> 6.95, 4096 x 4096 13.6 ->
+    // 12.4).  Long rows by the thousand are left as they were: the registers cost residency there (8192 x 8192 42.6 -> 44.4).
+    u32x4 const zero = {0u, 0u, 0u, 0u};
+    u32x4 v[CHUNKS], gam[CHUNKS], sca[CHUNKS];
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i)
     {
         int const piece = threadIdx.x + i * 256;
-        v[i] = piece < n8 ? *reinterpret_cast<u32x4 const*>(src + (long) piece * 8) : u32x4{0u, 0u, 0u, 0u};
+        bool const in = piece < n8;
+        v[i] = in ? *reinterpret_cast<u32x4 const*>(src + (long) piece * 8) : zero;
+        if constexpr (AHEAD)
+        {
+            gam[i] = in ? static_cast<u32x4 const*>(gamma)[piece] : zero;
+            sca[i] = in && scale ? static_cast<u32x4 const*>(scale)[piece] : zero;
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i)
+    {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
         {
@@ -59,9 +73,8 @@ __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void c
     __syncthreads();
     float const inv = __frsqrt_rn((part[0] + part[1] + part[2] + part[3]) / (float) k + eps);
 
-    auto finish = [&](u32x4 w, int piece)
+    auto finish = [&](u32x4 w, int piece, u32x4 g, u32x4 sc)
     {
-        u32x4 const g = static_cast<u32x4 const*>(gamma)[piece];
         u32x4 const b = beta ? static_cast<u32x4 const*>(beta)[piece] : u32x4{0u, 0u, 0u, 0u};
         u32x4 y;
 #pragma unroll
@@ -77,7 +90,6 @@ __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void c
         }
         if (scale)
         {
-            u32x4 const sc = static_cast<u32x4 const*>(scale)[piece];
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 y[r] = E::mul2(y[r], sc[r]);
@@ -99,11 +111,17 @@ __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void c
     for (int i = 0; i < CHUNKS; ++i)
     {
         int const piece = threadIdx.x + i * 256;
+        if constexpr (!AHEAD)
+        {
+            gam[i] = piece < n8 ? static_cast<u32x4 const*>(gamma)[piece] : zero;
+            sca[i] = piece < n8 && scale ? static_cast<u32x4 const*>(scale)[piece] : zero;
+        }
         if (piece < n8)
-            finish(v[i], piece);
+            finish(v[i], piece, gam[i], sca[i]);
     }
     for (int piece = threadIdx.x + CHUNKS * 256; piece < n8; piece += 256)
-        finish(*reinterpret_cast<u32x4 const*>(src + (long) piece * 8), piece);
+        finish(*reinterpret_cast<u32x4 const*>(src + (long) piece * 8), piece, static_cast<u32x4 const*>(gamma)[piece],
+            scale ? static_cast<u32x4 const*>(scale)[piece] : zero);
 }
 
 template <int DT, bool TO_FP8>
@@ -112,12 +130,17 @@ static void launch_chunks(void* out, void const* x, void const* gamma, void cons
 {
     dim3 grid((unsigned) m), block(256);
     int const pieces_per_thread = (k / 8 + 255) / 256;
+    bool const few = m <= 1024; // no more than four workgroups a CU
     if (pieces_per_thread <= 2)
-        hipLaunchKernelGGL((rmsnorm_prequant_kernel<DT, TO_FP8, 2>), grid, block, 0, s, out, x, gamma, beta, scale, eps, k);
+        hipLaunchKernelGGL((rmsnorm_prequant_kernel<DT, TO_FP8, 2, true>), grid, block, 0, s, out, x, gamma, beta, scale, eps, k);
+    else if (pieces_per_thread <= 4 && few)
+        hipLaunchKernelGGL((rmsnorm_prequant_kernel<DT, TO_FP8, 4, true>), grid, block, 0, s, out, x, gamma, beta, scale, eps, k);
     else if (pieces_per_thread <= 4)
-        hipLaunchKernelGGL((rmsnorm_prequant_kernel<DT, TO_FP8, 4>), grid, block, 0, s, out, x, gamma, beta, scale, eps, k);
+        hipLaunchKernelGGL((rmsnorm_prequant_kernel<DT, TO_FP8, 4, false>), grid, block, 0, s, out, x, gamma, beta, scale, eps, k);
+    else if (few)
+        hipLaunchKernelGGL((rmsnorm_prequant_kernel<DT, TO_FP8, 8, true>), grid, block, 0, s, out, x, gamma, beta, scale, eps, k);
     else
-        hipLaunchKernelGGL((rmsnorm_prequant_kernel<DT, TO_FP8, 8>), grid, block, 0, s, out, x, gamma, beta, scale, eps, k);
+        hipLaunchKernelGGL((rmsnorm_prequant_kernel<DT, TO_FP8, 8, false>), grid, block, 0, s, out, x, gamma, beta, scale, eps, k);
 }
 
 int launch_rmsnorm_prequant(void* out, void const* x, void const* gamma, void const* beta, void const* scale, float eps,
