@@ -604,9 +604,8 @@ int launch_w4a8_rt(GemmParams const& gp, int rt, hipStream_t s)
     }
 }
 
-int launch_gemm_w4a8(MatmulProblem const& p, void* stream)
+int launch_gemm_w4a8(MatmulProblem const& p, GemmPlan const& plan, void* stream)
 {
-    GemmPlan const plan = plan_gemm_w4a8(p.m, p.n, p.k);
     GemmParams gp;
     gp.act = p.act;
     gp.weight = p.weight;
