@@ -9,6 +9,9 @@ tensors made by ops.preprocess_weights_for_mixed_gemm, moved to the GPU.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
+import os
+import warnings
 
 import torch
 
@@ -26,9 +29,28 @@ INT8, INT4 = 1, 2
 BIAS, ZERO, PRE_QUANT_SCALE, FP8_ALPHA, INT8_WEIGHT = 1, 2, 4, 8, 16
 
 
-# A call outside a graph is bound by this file: one row of 4096 x 4096 takes the GPU 4 us and took the host 12.8 (9.8 now)
-# before pointers went to ctypes as plain integers, the stream handle came without a Stream object, device and layout were
-# asked with two attribute reads per tensor and the argument block was filled by position.
+# A call outside a graph is bound by the host: one row of 4096 x 4096 takes the GPU 4 us.  host/call.cpp does the plain case
+# of woq_matmul_raw in native code; what follows here is every other case, and all of them where it is not built.
+# (12.8 us a call before pointers went to ctypes as plain integers, the stream handle came without a Stream object, device
+# and layout were asked with two attribute reads per tensor and the argument block was filled by position; 9.5 ... 10.8 after, 5.4 natively.)
+def _load_native_call():
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "woq_call.so")
+    if not os.path.exists(path):
+        return None
+    spec = importlib.util.spec_from_file_location("woq_call", path)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except ImportError as e:  # built against another torch
+        warnings.warn("%s does not load (%s): matmul calls go through Python. Run build.py again." % (path, e))
+        return None
+    module.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (lib.woq_matmul, lib.woq_workspace_bytes)))
+    return module.matmul
+
+
+_native_matmul = _load_native_call()
+
+
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
@@ -60,6 +82,14 @@ def woq_matmul_raw(act, pre_quant_scale, weight, scales, zeros, bias, *, n: int,
     """One call of woq_matmul.  `act` is [..., k]; returns [..., n].  With `static_scratch` the call goes
     through woq_matmul_static: no workspace is allocated or passed, the library's own device array is
     used (pass `out` as well and the call allocates nothing at all)."""
+    if _native_matmul is not None and regime == 0 and workspace is None and out is None and not static_scratch \
+            and out_dtype is not None:
+        result = _native_matmul(act, pre_quant_scale, weight, scales, zeros, bias, n, k, group_size, quant_algo, alpha,
+                                _WOQ_DT.get(out_dtype, -1))
+        if result is not None:
+            if type(result) is int:
+                check(result)
+            return result
     _require_gpu(act, pre_quant_scale, weight, scales, zeros, bias, workspace, out)
     out_dtype = out_dtype or (act.dtype if act.dtype != torch.float8_e4m3fn else scales.dtype)
     if act.shape[-1] != k:
