@@ -92,9 +92,13 @@ bool pick_mid_one_tile(MatmulProblem const& p, size_t room, MidPlan& plan)
 // zeros; us, old -> new): 4096 x 4096 at 32 / 48 / 64 / 96 / 160 rows 10.5 -> 7.9 / 14.2 -> 9.6 / 15.7 -> 10.2 / 18.7 ->
 // 10.6 / 20.8 -> 13.6; 4096 x 6144 at 48 rows 16.0 -> 10.7; 14336 x 4096 19.2 -> 17.6; 4096 x 28672 at 32 / 48 rows
 // 20.5 -> 20.2 / 27.5 -> 23.7, at 64 rows slower (30 -> 36): the wide matrices keep the tiled kernels from there on.
-// `room`: bytes its float32 slabs may take.
+// Several workgroups of three or four row tiles share the weights beyond 64 rows; up to 512 rows that still beats the K splits
+// of the tiled kernels on narrow matrices: 2048 x 2048 at 176 / 256 / 512 rows 14 -> 10.5 / 16 -> 10.8 / 19 ... 22 -> 11 ... 13,
+// 4096 x 4096 at 208 / 256 rows int8 20.0 -> 15.6 / 22.9 -> 16.6, int4 per-channel 20.6 -> 15.0 / 20.7 -> 15.4, group 128 at 176
+// rows 21.0 -> 14.7 (profiles/mid_m_more_rows.csv: 196 problems of 144 ... 512 rows, 6 % on average over all of them).
+// `room`: bytes its float32 slabs may take.  `other_exact`: the other kernel is the exact-dequantize one.
 // WOQ_MID_SHAPE="rt,ns,waves,splits" forces it where it can run, "0" switches it off.
-bool pick_mid_shape(MatmulProblem const& p, double other_us, size_t room, MidPlan& plan)
+bool pick_mid_shape(MatmulProblem const& p, double other_us, size_t room, MidPlan& plan, bool other_exact = false)
 {
     EnvOverrides const& env = env_overrides();
     // (activations that do not start on 16 bytes stay with kernels that load them to registers: the DMA moves 16-byte pieces)
@@ -108,13 +112,21 @@ bool pick_mid_shape(MatmulProblem const& p, double other_us, size_t room, MidPla
     }
     if (!p.built_in_choice || p.m > kMidMaxM)
         return false;
+    if (p.m > 160 && (p.n < 2048 || p.k < 2048)) // (nothing smaller is among the timings of that many rows)
+        return false;
     if (p.m <= 16)
         return pick_mid_one_tile(p, room, plan);
-    double const t = best_mid_plan(p.m, p.n, p.k, p.bits, p.group_size, room, plan);
+    // fp16 operands of int8 weights carry 1024 + u, which costs activations of one sign precision that grows with the length
+    // of a float32 sum (4096 x 4096, 256 rows, error against 64 bits: exact 2.07e-4, eight wavefronts 2.10e-4, deferred-scale
+    // 2.16e-4, four wavefronts 2.19e-4; without a mean all are at 2.07e-4): no rows are moved to a longer sum than they had
+    bool const long_sums = p.m > 160 && p.bits == 8 && p.act_dtype == WOQ_FP16;
+    if (long_sums && other_exact)
+        return false;
+    double const t = best_mid_plan(p.m, p.n, p.k, p.bits, p.group_size, room, plan, long_sums);
     // (0.88: of 95 measured problems of 17 ... 160 rows the choice costs 2 % on average against the better of the two and
     // leaves three slower than the other kernel, by 1, 5 and 7 %; at 0.85 one of those is left, by 1 %, and problems that gain
-    // 6 ... 17 % go with the two; at 1.0 a few lose 10 %)
-    return t > 0 && t < 0.88 * other_us;
+    // 6 ... 17 % go with the two; at 1.0 a few lose 10 %.  Above 160 rows 0.85 leaves none slower.)
+    return t > 0 && t < (p.m > 160 ? 0.85 : 0.88) * other_us;
 }
 
 int launch_mid(MatmulProblem const& p, MidPlan const& plan, void* stream)
@@ -133,7 +145,7 @@ int launch_gemm(MatmulProblem const& p, void* stream)
     {
         GemmPlan const plan = planned_gemm(p.m, p.n, p.k, p.bits, p.group_size, room, false, p.contract);
         MidPlan mid;
-        bool const is_mid = pick_mid_shape(p, plan.cost_us, room, mid);
+        bool const is_mid = pick_mid_shape(p, plan.cost_us, room, mid, !plan.skinny);
         if ((is_mid ? split_partial_bytes(p.m, p.n, mid.splits) : plan.ws_bytes) > given && room > given)
             continue; // less workspace than woq_workspace_bytes asks for: the cheapest plan that fits it
         return is_mid ? launch_mid(p, mid, stream) : launch_gemm_planned(p, plan, stream);
