@@ -64,17 +64,6 @@ struct Elem<WOQ_BF16>
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
     }
 
-    // the same on blocks of 32 x 32 x 16: twice the work for one issue slot
-    static __device__ __forceinline__ void mma_acc(u32x4 a, u32x4 b, f32x16& c)
-    {
-        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-    }
-
-    static __device__ __forceinline__ void mma_first(u32x4 a, u32x4 b, f32x16& c)
-    {
-        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
-    }
-
     static __device__ __forceinline__ float lo(uint32_t pair)
     {
         return bit_cast<float>(pair << 16);
@@ -136,17 +125,6 @@ struct Elem<WOQ_FP16>
     static __device__ __forceinline__ void mma_first(u32x4 a, u32x4 b, f32x4& c)
     {
         asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
-    }
-
-    // the same on blocks of 32 x 32 x 16: twice the work for one issue slot
-    static __device__ __forceinline__ void mma_acc(u32x4 a, u32x4 b, f32x16& c)
-    {
-        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-    }
-
-    static __device__ __forceinline__ void mma_first(u32x4 a, u32x4 b, f32x16& c)
-    {
-        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
     }
 
     static __device__ __forceinline__ float lo(uint32_t pair)

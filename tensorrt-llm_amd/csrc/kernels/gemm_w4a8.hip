@@ -34,8 +34,8 @@ namespace woq
 {
 
 // PERSIST (256-row tiles, whole K, bf16 output, no bias): one workgroup per CU walks tiles b, b + grid, ...
-// as the 16-bit prefill kernel does (gemm_kernel.h): the last two steps of a tile already request the
-// first weights and the first A tile of the next one, and a finished tile's outputs are read out of
+// as the 16-bit prefill kernel does (gemm_kernel.h): the last steps of a tile already request the
+// first weights and A tiles of the next one, and a finished tile's outputs are read out of
 // the accumulators, scaled, packed and stored right before the matrix instruction that starts each
 // block's new sum.  The 8 us or so that a tile spends outside its main loop (first loads, the
 // conversion of the first operand set, 128 KiB of stores, the relaunch) weigh twice as much here as
@@ -131,8 +131,8 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
             x.wlane[cb] = ((uint32_t) strip * (uint32_t) p.k_tiles * 64u + (uint32_t) (kh * 32 + lane_col)) * 16u;
             x.sc_lane[cb] = (uint32_t) (strip * 16 + lane_col) * 2u;
         }
-        // A tile -> LDS: wavefront w moves pairs w, w+4, ...: piece i is pair f = w + 4i = half w % 2 of
-        // row tile 2i + w / 2
+        // A tile -> LDS: wavefront w moves pairs w, w+8, ...: piece i is pair f = w + 8i = half w % 2 of
+        // row tile 4i + w / 2
         x.dma_lane_base = (uint32_t) (tm_ * BM + (wave / 2) * 16 + (lane >> 2)) * (uint32_t) K
             + (uint32_t) ((wave % 2) * 64 + (((lane & 3) ^ ((lane >> 4) & 3)) * 16));
         x.oob = valid ? 0u : 0x80000000u;
@@ -198,7 +198,7 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
     // The operands of one instruction along K (8 registers) are all there is of converted weights: while the row blocks
     // are multiplied with those of ki = 0, ki = 1 of the same step is converted, meanwhile ki = 0 of the next step.
     // Conversion is a look-up (w4a8_common.h): a (group, column) has sixteen possible e4m3 results; the two lanes that feed
-    // a column each compute eight of them - the same FMA and saturating conversion as dequant2_fp8, so the bytes are
+    // a column each compute eight of them - the same FMA and saturating conversion as dequant4_fp8, so the bytes are
     // identical, with zero-points or without - and exchange them.  15 instructions per eight weights against 21 issue slots
     // of the arithmetic form (the conversion instruction takes two).
     constexpr int A_AHEAD = 2;

@@ -7,51 +7,10 @@
 namespace woq
 {
 
-// elements 4h+2p, 4h+2p+1 of slab dword `w` -> 2 e4m3 bytes in 16-bit word p of `old` (a dword of
-// the B operand holds elements 4h .. 4h+3 in order; the other word is kept).
-// CLAMP = false is for kernels that run with fp8_saturation_on(): the conversion instruction then
-// saturates by itself and the clamp (a quarter of the instructions) is not needed.
-// With zero-points the weight is fma(q, s, z) on the two's-complement nibble.  Without them
-// q * s = fma(u, s, -8 s) on the stored nibble u = q + 8: -8 s is exact, so this is the same
-// single rounding, and u comes out of a byte-to-float conversion with no sign extension.
-template <bool ZERO, bool CLAMP = true>
-__device__ __forceinline__ uint32_t dequant2_fp8(uint32_t old, uint32_t w, int h, int p, float s, float z)
-{
-    float v0, v1;
-    // elements e0 = 4h + 2p and e0 + 1 sit in nibble slots e0/2 and 4 + e0/2
-    if constexpr (ZERO)
-    {
-        // q/16 straight from the nibble (see int4_pair_sixteenths), times 16 s: the same rounding.
-        // Slots e0/2 and 4 + e0/2 are the low nibbles of bytes h and h+2 of t (p = 0) or t >> 4 (p = 1).
-        uint32_t const t = w ^ 0x88888888u; // biased -> two's complement nibbles
-        uint32_t const src = p == 0 ? t : t >> 4;
-        float const s16 = 16.f * s;
-        v0 = __builtin_fmaf(cvt_off_f32_i4_byte(src, h), s16, z);
-        v1 = __builtin_fmaf(cvt_off_f32_i4_byte(src, h + 2), s16, z);
-    }
-    else
-    {
-        // slots e0/2 and 4 + e0/2 are bytes h and h+2 of the even-nibble word (p = 0) or of the
-        // odd-nibble word (p = 1).  The masked word is made opaque so that the byte-to-float
-        // conversions read it (the compiler would otherwise extract each 4-bit field from w).
-        uint32_t m = (p == 0 ? w : (w >> 4)) & 0x0F0F0F0Fu;
-        asm volatile("" : "+v"(m));
-        float const m8s = -8.f * s;
-        v0 = __builtin_fmaf((float) ((m >> (8 * h)) & 0xFF), s, m8s);
-        v1 = __builtin_fmaf((float) ((m >> (8 * h + 16)) & 0xFF), s, m8s);
-    }
-    if constexpr (CLAMP) // saturation to +-448 in software; off when the conversion itself saturates
-    {
-        v0 = clamp_e4m3(v0);
-        v1 = clamp_e4m3(v1);
-    }
-    return p == 0 ? (uint32_t) __builtin_amdgcn_cvt_pk_fp8_f32(v0, v1, (int) old, false)
-                  : (uint32_t) __builtin_amdgcn_cvt_pk_fp8_f32(v0, v1, (int) old, true);
-}
-
-// One dword of the B operand (elements 4h .. 4h+3 of slab dword `w`), same arithmetic
+// One dword of the B operand: elements 4h .. 4h+3 of slab dword `w` -> 4 e4m3 bytes, each fma(q, s, z) rounded once
 // (`nib`: nibble_consts<WOQ_FP16>(), the mask 0x000F000F and 1024 as a pair of halves in registers).  CLAMP =
-// false leaves the saturation to +-448 out: for callers that know 8|s| + |z| stays below it.
+// false leaves the saturation to +-448 out: for callers that know 8|s| + |z| stays below it, or that run with
+// fp8_saturation_on().
 template <bool ZERO, bool CLAMP>
 __device__ __forceinline__ uint32_t dequant4_fp8(uint32_t w, int h, float s, float z, NibbleConsts const& nib)
 {
@@ -246,20 +205,9 @@ inline uint32_t w4a8_scale_row_magic(int group_size)
 typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
-// c += a x b (32 e4m3 values per lane each), accumulator tied to one AGPR quad (see Elem::mma_acc)
-__device__ __forceinline__ void mma_fp8_acc(u32x8 a, u32x8 b, f32x4& c)
-{
-    asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-
-// c = a x b: the first product of a new sum (the old value of c is dead: no input operand for it)
-__device__ __forceinline__ void mma_fp8_first(u32x8 a, u32x8 b, f32x4& c)
-{
-    asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
-}
-
-// the same on blocks of 32 x 32 x 64: twice the work for one issue slot.  AGPR: accumulators in the upper half of the
-// register file; the old value is an operand of the first product too, so that both name the same registers
+// c += a x b (32 e4m3 values per lane each) on blocks of 32 x 32 x 64: twice the work of 16 x 16 x 128 for one issue slot.
+// AGPR: accumulators in the upper half of the register file.  mma_fp8_first: the first product of a new sum (c = a x b; in
+// ordinary registers c is named as an operand all the same, so that sum and first product keep one register block)
 template <bool AGPR>
 __device__ __forceinline__ void mma_fp8_acc(u32x8 a, u32x8 b, f32x16& c)
 {

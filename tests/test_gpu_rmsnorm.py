@@ -71,3 +71,16 @@ def test_rmsnorm_feeds_the_matmul(pkg, oracle, dev):
                                 quant_algo=F.FP8_ALPHA | F.PRE_QUANT_SCALE, alpha=prob["alpha"], out_dtype=torch.bfloat16)
     torch.cuda.synchronize()
     assert torch.equal(fused, two_step)
+
+
+@pytest.mark.parametrize("k", [4096, 4104])
+def test_rmsnorm_rows_do_not_depend_on_their_number(pkg, oracle, dev, k):
+    """Beyond 1024 rows of more than 4096 elements the tables are read behind the sum of squares: the bits of the launch
+    that requests them with the row."""
+    F = pkg.functional
+    x, gamma, b, s = _case(oracle, 1030, k, "bf16", True, True, seed=k)
+    xs, rest = to_dev(x, "bf16", dev), [to_dev(gamma, "bf16", dev), to_dev(s, "bf16", dev), 1e-5, to_dev(b, "bf16", dev)]
+    for out_type in (None, torch.float8_e4m3fn):
+        many = F.rmsnorm_prequant(xs, *rest, out_type).float()
+        few = torch.cat([F.rmsnorm_prequant(part, *rest, out_type).float() for part in (xs[:1024], xs[1024:])])
+        assert torch.equal(many, few)

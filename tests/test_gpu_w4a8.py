@@ -430,3 +430,58 @@ def test_w4a8_multirow_kernel_rule_and_exact_rows(pkg, oracle, dev):
             w8 = oracle.dequantize(q, s, z, G, "fp8")
             assert np.abs(w8).max() == 448.0
             assert (out == oracle.round_f16(w8[hot])).all(), (M, K, N, z is not None)
+
+
+@pytest.mark.parametrize("rt", [4, 8, 16])
+@pytest.mark.parametrize("with_zeros", [False, True])
+@pytest.mark.parametrize("M,N,group", [(17, 272, 128), (129, 528, 256), (257, 256, 384)])
+def test_w4a8_tiled_every_tile_count(pkg, oracle, dev, woq_env, rt, with_zeros, M, N, group):
+    """Every height over one to nine tile rows of K (the loop runs three ahead over four buffers), one slice and slices of
+    which the last are short or empty: sums of each row of K once, scales of the right group, the same bits twice.  Sparse
+    one-hot rows of activations, so that each output is one e4m3 weight times alpha, exactly."""
+    woq_env(WOQ_GEMM_RT=str(rt))
+    for tiles in range(1, 10):
+        K, rows = 128 * tiles, -(-tiles * 128 // group)
+        rng = np.random.default_rng(100 * tiles + rt)
+        act = np.zeros((M, K), np.float32)
+        hot = (37 * np.arange(M) + 11 * tiles) % K
+        act[np.arange(M), hot] = 1.0
+        prob = dict(q=rng.integers(-8, 8, size=(K, N)).astype(np.int8), act=act, alpha=0.5,
+                    scales=oracle.round_f16(np.exp(rng.uniform(-2, 3, (rows, N))).astype(np.float32)),
+                    pre_quant_scale=np.ones(K, np.float32))
+        zeros = oracle.round_f16((rng.standard_normal((rows, N)) * 20).astype(np.float32)) if with_zeros else None
+        w8 = oracle.dequantize(prob["q"], prob["scales"], zeros, group, "fp8")
+        for splits in sorted({1, min(3, tiles), tiles}):
+            woq_env(WOQ_GEMM_SPLITS=str(splits))
+            out, _ = _run(pkg, oracle, dev, prob, M, K, N, "fp16", zeros=zeros, direct_fp8=True, regime=GEMM, group=group)
+            assert "w4a8 rt=%d splits=%d" % (rt, splits) in _launch(pkg), _launch(pkg)
+            assert (out == oracle.round_f16(0.5 * w8[hot])).all(), (tiles, splits)
+
+
+def test_w4a8_few_rows_on_the_tiled_kernel(pkg, oracle, dev):
+    """Nine to 32 rows of a long product run on the tiled kernel; its workspace stays the one that the size query
+    names, a smaller one is refused as before, and the library's own device array gives the same bits."""
+    F = pkg.functional
+    K, N = 14336, 4096
+    for M, tiled in ((8, False), (9, None), (32, True)):
+        prob = oracle.make_w4a8_problem(M, K, N, seed=M, out_dtype="bf16")
+        out, ref = _run(pkg, oracle, dev, prob, M, K, N, "bf16", direct_fp8=True)
+        assert tiled is None or ("gemm w4a8" in _launch(pkg)) == tiled, _launch(pkg)
+        assert _perr(oracle, out, ref, prob) < TOL
+        if M < 32:
+            continue
+        a8 = torch.from_numpy(oracle.apply_per_channel_scale(prob["act"], prob["pre_quant_scale"], "bf16", "fp8")).to(dev)
+        operands = (a8.to(torch.float8_e4m3fn), None, preprocess(pkg, oracle, prob["q"], 4, torch.float8_e4m3fn).to(dev),
+                    to_dev(prob["scales"], "fp16", dev), None, None)
+        how = dict(n=N, k=K, group_size=128, quant_algo=F.FP8_ALPHA, alpha=prob["alpha"], out_dtype=torch.bfloat16)
+        same = F.woq_matmul_raw(*operands, static_scratch=True, **how)
+        torch.cuda.synchronize()
+        assert (same.float().cpu().numpy() == out).all(), _launch(pkg)
+        need = pkg._lib.lib.woq_workspace_bytes(M, N, K, F.FP8_ALPHA, F._WOQ_DT[torch.float8_e4m3fn])
+        for given in (need, 4 * need):
+            ws = torch.full((given,), 0x7F, dtype=torch.uint8, device=dev)
+            got = F.woq_matmul_raw(*operands, workspace=ws, **how)
+            torch.cuda.synchronize()
+            assert (got.float().cpu().numpy() == out).all(), (_launch(pkg), given)
+        with pytest.raises(pkg._lib.WoqError, match="workspace of %d bytes required" % need):
+            F.woq_matmul_raw(*operands, workspace=ws[:need - 1], **how)
