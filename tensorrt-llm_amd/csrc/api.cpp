@@ -125,7 +125,8 @@ bool pick_mid_shape(MatmulProblem const& p, double other_us, size_t room, MidPla
     double const t = best_mid_plan(p.m, p.n, p.k, p.bits, p.group_size, room, plan, long_sums);
     // (0.88: of 95 measured problems of 17 ... 160 rows the choice costs 2 % on average against the better of the two and
     // leaves three slower than the other kernel, by 1, 5 and 7 %; at 0.85 one of those is left, by 1 %, and problems that gain
-    // 6 ... 17 % go with the two; at 1.0 a few lose 10 %.  Above 160 rows 0.85 leaves none slower.)
+    // 6 ... 17 % go with the two; at 1.0 a few lose 10 %.  Above 160 rows 0.85 leaves none
+    // of 196 slower by more than 4 %.)
     return t > 0 && t < (p.m > 160 ? 0.85 : 0.88) * other_us;
 }
 

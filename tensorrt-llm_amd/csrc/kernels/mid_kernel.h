@@ -1,4 +1,4 @@
-// 8 to 160 rows without a barrier in the main loop: the rows between the decode kernels and the tall prefill tiles
+// 8 to 512 rows without a barrier in the main loop: the rows between the decode kernels and the tall prefill tiles
 // (the reference covers them with CUTLASS tiles of 16 ... 64 rows and split-K,
 // cpp/tensorrt_llm/kernels/cutlass_kernels/cutlass_heuristic.cpp:59-140).
 //
