@@ -83,11 +83,13 @@ __global__ void __launch_bounds__(256) probe_mfma_kernel(float* sink, int iters)
                 asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc32[i]) : "v"(a4[i & 3]), "v"(b4[i & 3]));
         }
         mma_drain();
-        asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
         float s = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
+        {
+            asm volatile("" : "+a"(acc32[i])); // (what is read stays behind the drain)
             s += acc32[i][0];
+        }
         sink[(blockIdx.x * 256 + threadIdx.x) & 511] = s;
         return;
     }
