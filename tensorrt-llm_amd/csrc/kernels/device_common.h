@@ -49,10 +49,11 @@ struct Elem<WOQ_BF16>
 
     // c += a x b with the accumulator tied to ONE AGPR quad.  The builtin leaves destination and
     // addend independent; with 256 live accumulator registers the allocator then renames them
-    // along the K loop and pays for it with hundreds of AGPR<->VGPR copies per step.  (A and B
-    // operands written by ordinary VALU instructions need no software wait states before an
-    // MFMA; the result must not be read by VALU code until the MFMA has drained - see
-    // mma_drain().)
+    // along the K loop and pays for it with hundreds of AGPR<->VGPR copies per step.  The compiler does not see
+    // a matrix instruction in here and keeps no distance for it: two wait states between the vector
+    // instruction that writes an A or B operand and this one are up to the kernel's schedule, and the result must not
+    // be touched by other instructions before the MFMA has drained - see mma_drain().  (Both are checked on the
+    // built code: tests/test_matrix_hazards.py.)
     static __device__ __forceinline__ void mma_acc(u32x4 a, u32x4 b, f32x4& c)
     {
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
@@ -174,7 +175,7 @@ __device__ __forceinline__ void mma_drain()
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 }
 
-// The same without holding back memory operations, for inside a main loop: 20 wait states, one more than a vector
+// The same without holding back memory operations, for inside a main loop: the 20 wait states that a vector
 // instruction needs behind a 16-pass matrix instruction.
 __device__ __forceinline__ void mma_settle()
 {

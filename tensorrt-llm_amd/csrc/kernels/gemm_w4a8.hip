@@ -202,6 +202,8 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
     // identical, with zero-points or without - and exchange them.  15 instructions per eight weights against 21 issue slots
     // of the arithmetic form (the conversion instruction takes two).
     constexpr int A_AHEAD = 2;
+    // Two row blocks: the conversions end right in front of the next matrix instruction, which reads them
+    constexpr bool B_JUST_WRITTEN = RB <= 2;
     Fp8LookupConsts const lut = fp8_lookup_consts();
     f16x2 qv[4]; // the lane's eight signed values 8 kh - 8 ... 8 kh - 1, as halves for mixed-precision FMAs
 #pragma unroll
@@ -324,14 +326,14 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
             // (the split-K variant keeps the plain orientation: its float32 stores cover 128 consecutive
             // bytes per row and instruction)
             if constexpr (SPLITK)
-                mma_fp8_acc<RT == 16>(a_cur, b[ki], acc[rb][0]);
+                mma_fp8_acc<RT == 16, B_JUST_WRITTEN>(a_cur, b[ki], acc[rb][0]);
             else if (FIRST && ki == 0)
             {
                 store_block(rb, 0); // the previous tile's sums leave right before the block starts the new tile's
                 mma_fp8_first<RT == 16>(b[ki], a_cur, acc[rb][0]);
             }
             else
-                mma_fp8_acc<RT == 16>(b[ki], a_cur, acc[rb][0]);
+                mma_fp8_acc<RT == 16, B_JUST_WRITTEN>(b[ki], a_cur, acc[rb][0]);
             // behind the MFMA its share of the conversions, half units at a time: a wavefront issues in order, so the
             // VALU work has to sit between the matrix instructions to run under them
             BStage const& src = ki == 0 ? st : st_next;

@@ -207,11 +207,17 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 
 // c += a x b (32 e4m3 values per lane each) on blocks of 32 x 32 x 64: twice the work of 16 x 16 x 128 for one issue slot.
 // AGPR: accumulators in the upper half of the register file.  mma_fp8_first: the first product of a new sum (c = a x b; in
-// ordinary registers c is named as an operand all the same, so that sum and first product keep one register block)
-template <bool AGPR>
+// ordinary registers c is named as an operand all the same, so that sum and first product keep one register block).
+// WAIT: two wait states in front, which an operand needs that a vector instruction has just written (Elem::mma_acc).
+template <bool AGPR, bool WAIT>
 __device__ __forceinline__ void mma_fp8_acc(u32x8 a, u32x8 b, f32x16& c)
 {
-    if constexpr (AGPR)
+    if constexpr (WAIT)
+    {
+        static_assert(!AGPR, "not needed there: other instructions stand in between");
+        asm volatile("s_nop 1\n\tv_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+    }
+    else if constexpr (AGPR)
         asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     else
         asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));

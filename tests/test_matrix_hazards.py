@@ -138,5 +138,5 @@ def test_built_kernels_keep_the_wait_states(pkg, tmp_path):
     parts = sorted(tmp_path.glob("*gfx950*"))
     assert parts, "no device code in %s" % pkg.lib_path()
     with concurrent.futures.ProcessPoolExecutor(4) as pool:
-        found = [h for h in sum(pool.map(_hazards_of, parts), []) if "result" in h[3]]
+        found = sum(pool.map(_hazards_of, parts), [])
     assert not found, "%d hazards, the first: %s" % (len(found), found[:8])
