@@ -77,28 +77,35 @@ def _compile(src: str) -> str:
     return obj
 
 
-def build_call(verbose: bool = True) -> None:
-    """woq_call.so: the native form of functional.py's ordinary call, against the torch that is installed (libwoq.so
-    itself does without torch)."""
+def build_call(verbose: bool = True) -> bool:
+    """woq_call.so: the native form of functional.py's ordinary call, against the torch that is installed.  An extra:
+    libwoq.so does without torch, and functional.py without this file - where it cannot be built (a torch for other
+    hardware, no g++, no headers) that is said, and none of an earlier build is left behind."""
+    out = os.path.join(HERE, "woq_call.so")
+    if os.path.exists(out):
+        os.remove(out)
     try:
+        import sysconfig
         import torch
         from torch.utils.cpp_extension import include_paths
-    except ImportError:
-        print("no torch: woq_call.so (calls from Python without its overhead) is not built")
-        return
-    import sysconfig
-    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    out = os.path.join(HERE, "woq_call.so")
-    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
-    cmd += ["-I" + p for p in include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include"]]
-    cmd += [os.path.join(HERE, "host", "call.cpp"), "-o", out, "-L" + torch_lib]
-    cmd += ["-l" + n for n in ("torch_python", "torch", "torch_cpu", "torch_hip", "c10", "c10_hip")]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError("g++ failed for host/call.cpp:\n" + r.stderr)
+        torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+        cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+               "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+        cmd += ["-I" + p for p in include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include"]]
+        cmd += [os.path.join(HERE, "host", "call.cpp"), "-o", out, "-L" + torch_lib]
+        cmd += ["-l" + n for n in ("torch_python", "torch", "torch_cpu", "torch_hip", "c10", "c10_hip")]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        problem = (r.stderr or "g++ failed") if r.returncode != 0 else ""
+    except (ImportError, AttributeError, OSError) as e:
+        problem = str(e)
+    if problem:
+        sys.stderr.write("woq_call.so (matmul calls from Python without Python's overhead) is not built:\n%s\n" % problem)
+        if os.path.exists(out):
+            os.remove(out)
+        return False
     if verbose:
         print("built %s" % out)
+    return True
 
 
 def build_lib(jobs: int | None = None, verbose: bool = True) -> str:
@@ -107,14 +114,14 @@ def build_lib(jobs: int | None = None, verbose: bool = True) -> str:
     jobs = jobs or min(8, os.cpu_count() or 1)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         objs = list(ex.map(_compile, srcs))
-    if os.path.basename(LIB) == "libwoq.so":
-        build_call(verbose)
     cmd = [HIPCC, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", LIB] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
     if verbose:
         print("built %s from %d translation units" % (LIB, len(srcs)))
+    if os.path.basename(LIB) == "libwoq.so":
+        build_call(verbose)
     return LIB
 
 
