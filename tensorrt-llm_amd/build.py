@@ -90,7 +90,7 @@ def build_call(verbose: bool = True) -> bool:
         from torch.utils.cpp_extension import include_paths
         torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
         cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-               "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+               "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, '-DWOQ_CALL_TORCH="%s"' % torch.__version__]
         cmd += ["-I" + p for p in include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include"]]
         cmd += [os.path.join(HERE, "host", "call.cpp"), "-o", out, "-L" + torch_lib]
         cmd += ["-l" + n for n in ("torch_python", "torch", "torch_cpu", "torch_hip", "c10", "c10_hip")]

@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import sys
 import warnings
 
 import torch
@@ -33,15 +34,18 @@ BIAS, ZERO, PRE_QUANT_SCALE, FP8_ALPHA, INT8_WEIGHT = 1, 2, 4, 8, 16
 # of woq_matmul_raw in native code; what follows here is every other case, and all of them where it is not built.
 # (12.8 us a call before pointers went to ctypes as plain integers, the stream handle came without a Stream object, device
 # and layout were asked with two attribute reads per tensor and the argument block was filled by position; 9.5 ... 10.8 after, 5.4 natively.)
-def _load_native_call():
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "woq_call.so")
+def _load_native_call(path=os.path.join(os.path.dirname(os.path.abspath(__file__)), "woq_call.so")):
     if not os.path.exists(path):
         return None
+    here = (str(torch.__version__), lib.woq_abi_version(), *sys.version_info[:2])
     spec = importlib.util.spec_from_file_location("woq_call", path)
     try:
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
-    except ImportError as e:  # built against another torch
+        built_for = module.built_for()
+        if built_for != here:  # its inlined code knows tensors and argument block by their layout
+            raise ImportError("built for torch %s, ABI %s, Python %s.%s; these are %s, %s, %s.%s" % (*built_for, *here))
+    except (ImportError, AttributeError) as e:  # (symbols of another torch, an older build)
         warnings.warn("%s does not load (%s): matmul calls go through Python. Run build.py again." % (path, e))
         return None
     module.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (lib.woq_matmul, lib.woq_workspace_bytes)))

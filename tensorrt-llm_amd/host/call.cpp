@@ -47,7 +47,7 @@ int dtype_of(at::ScalarType t)
 PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 {
     HANDLE_TH_ERRORS
-    if (nargs != 12 || at::impl::torch_function_mode_enabled())
+    if (!g_matmul || nargs != 12 || at::impl::torch_function_mode_enabled())
         Py_RETURN_NONE;
     at::Tensor const* t[6];
     for (int i = 0; i < 6; ++i)
@@ -127,6 +127,13 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs)
     END_HANDLE_TH_ERRORS
 }
 
+// What this file was compiled against: the torch whose tensors it looks into, the argument block of include/woq.h, Python.
+// A torch or a library of another build may load all the same and be laid out differently; the caller compares.
+PyObject* built_for(PyObject*, PyObject*)
+{
+    return Py_BuildValue("(siii)", WOQ_CALL_TORCH, WOQ_ABI_VERSION, PY_MAJOR_VERSION, PY_MINOR_VERSION);
+}
+
 // bind(address of woq_matmul, address of woq_workspace_bytes): the library that _lib.py loaded
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 {
@@ -145,7 +152,8 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 }
 
 PyMethodDef methods[] = {{"matmul", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(matmul)), METH_FASTCALL, nullptr},
-    {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(bind)), METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
+    {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(bind)), METH_FASTCALL, nullptr},
+    {"built_for", built_for, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "woq_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 } // namespace
 

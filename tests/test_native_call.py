@@ -24,6 +24,35 @@ def test_native_call_is_built(pkg):
     assert pkg.functional._native_matmul is not None
 
 
+@pytest.mark.parametrize("other", ["torch", "abi", "python"])
+def test_built_for_something_else(pkg, monkeypatch, other):
+    """A file that loads but was compiled against another torch, library interface or Python is not used."""
+    F = pkg.functional
+    if other == "torch":
+        monkeypatch.setattr(torch, "__version__", torch.__version__ + ".other")
+    elif other == "abi":
+        abi = F.lib.woq_abi_version()
+
+        class Lib:
+            woq_matmul, woq_workspace_bytes = F.lib.woq_matmul, F.lib.woq_workspace_bytes
+
+            @staticmethod
+            def woq_abi_version():
+                return abi + 1
+
+        monkeypatch.setattr(F, "lib", Lib)
+    else:
+        monkeypatch.setattr(F.sys, "version_info", (3, 99, 0, "final", 0))
+    with pytest.warns(UserWarning, match="matmul calls go through Python"):
+        assert F._load_native_call() is None
+
+
+def test_not_a_library(pkg, tmp_path):
+    (tmp_path / "woq_call.so").write_bytes(b"not one")
+    with pytest.warns(UserWarning, match="does not load"):
+        assert pkg.functional._load_native_call(str(tmp_path / "woq_call.so")) is None
+
+
 @pytest.mark.parametrize("change", ["cpu", "strided", "subclass", "dtype", "k", "n_args"])
 def test_not_for_the_native_path(pkg, change):
     """None: the Python path decides (on a machine without a GPU every tensor is refused there)."""
