@@ -23,6 +23,7 @@
 // Measured (bf16 output, group 128, no zero-points, us; before: four wavefronts of 64 columns, 16x16x128 instructions,
 // two buffers, arithmetic conversion): 4096 x 28672 at 64 / 1990 / 8192 rows 55.9 -> 26.8 / 234 -> 198 / 851 -> 737 (2.61
 // PFLOP/s), 8192 x 57344 at 128 / 256 rows 119 -> 69.6 / 116 -> 107, 4096 x 4096 at 1990 rows 54.3 -> 36.2 (128-row tiles).
+// With zero-points, on another box: 4096 x 28672 at 1990 / 8192 rows 255 -> 200 / 908 -> 753, 8192 x 57344 at 1024 rows 475 -> 393.
 // By step, 8192 x 57344 at 128 rows: 32x32x64 109, eight wavefronts 88, three steps ahead 75, look-up conversion 70.
 // What bounds it: 128-row tiles the conversions (140 issue slots of each wavefront a step beside 8 instructions of 64
 // cycles); 256-row ones the LDS (every wavefront reads the whole activation tile: 2048 + 256 cycles a step, as many as the
@@ -43,6 +44,14 @@ namespace woq
 constexpr int kW4a8Waves = 8;
 constexpr int kOneTile = 0, kPersistPairs = 1, kPersist = 2; // persistent forms: steps in pairs (any even K), in fours
 
+constexpr uint32_t kLdsReach = 0x10000; // of an LDS instruction's immediate offset
+template <bool UPPER>
+struct W4a8Buf // one activation tile in LDS
+{
+    static constexpr bool upper = UPPER;
+    u32x4* data;
+};
+
 template <int ODT, bool ZERO, int RT, bool SPLITK, int LOOP = kOneTile>
 __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm_w4a8_kernel(GemmParams p)
 {
@@ -58,10 +67,13 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
     constexpr int A_BYTES = BM * TK;   // e4m3: one byte per element
     static_assert(PAIRS % NW == 0 && CB == 1, "one column block a wavefront; fragment pairs spread evenly over the wavefronts");
 
-    __shared__ u32x4 a_buf0[A_BYTES / 16];
-    __shared__ u32x4 a_buf1[A_BYTES / 16];
-    __shared__ u32x4 a_buf2[A_BYTES / 16];
-    __shared__ u32x4 a_buf3[A_BYTES / 16];
+    __shared__ u32x4 a_lds0[A_BYTES / 16];
+    __shared__ u32x4 a_lds1[A_BYTES / 16];
+    __shared__ u32x4 a_lds2[A_BYTES / 16];
+    __shared__ u32x4 a_lds3[A_BYTES / 16];
+    constexpr bool UPPER = 4 * A_BYTES > (int) kLdsReach; // buffers 2 and 3 lie beyond what an LDS read's immediate offset reaches
+    W4a8Buf<false> const a_buf0{a_lds0}, a_buf1{a_lds1};
+    W4a8Buf<UPPER> const a_buf2{a_lds2}, a_buf3{a_lds3};
 
     // Tile of virtual block vb (the block index, or with PERSIST the block index plus a multiple of the
     // grid size, which is a multiple of 8): XCD-contiguous chunks of the tile order, m fastest inside
@@ -153,11 +165,11 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
     uint32_t const dma_piece_stride = (uint32_t) NW * 8u * (uint32_t) K;
     auto dma_base = [&](int kt, TileCtx const& x) -> uint32_t
     { return (x.dma_lane_base + (uint32_t) kt * (uint32_t) TK) | ((uint32_t) (KT - 1 - kt) & kOob) | x.oob; };
-    auto dma_piece = [&](auto* buf, uint32_t base, int i)
+    auto dma_piece = [&](auto buf, uint32_t base, int i)
     {
         int const f = wave + i * NW;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(act_rsrc,
-            (__attribute__((address_space(3))) void*) (reinterpret_cast<char*>(buf) + f * 1024), 16,
+            (__attribute__((address_space(3))) void*) (reinterpret_cast<char*>(buf.data) + f * 1024), 16,
             (int) (base + (uint32_t) i * dma_piece_stride), 0, 0, 0);
     };
     // Matrix instruction ki of a tile row covers slabs 2 ki and 2 ki + 1; lane (kh, row_in) supplies the 16 values
@@ -168,6 +180,20 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
 #pragma unroll
     for (int jj = 0; jj < 2; ++jj)
         a_lane_off[jj] = (uint32_t) ((row_in >> 4) * 2048 + ((row_in & 15) * 4 + ((jj * 2 + kh) ^ ((row_in >> 2) & 3))) * 16);
+
+    // The immediate offset of an LDS read reaches 64 KiB.  With 256-row tiles the buffers 2 and 3 lie beyond it, and the compiler,
+    // which does not split an offset, kept an address register for each of their 32 reads: 14 of them (with zero-points; ten
+    // without) in scratch memory, whose reloads waited for every request in flight.  These are the same offsets as seen
+    // from 64 KiB on, which it is not told (4096 x 28672 at 1990 / 8192 rows with zero-points 210 -> 200 / 788 -> 753 us, without
+    // 202 -> 198 / 763 -> 745)
+    uint32_t a_lane_upper[2];
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj)
+    {
+        a_lane_upper[jj] = a_lane_off[jj] + kLdsReach;
+        if constexpr (UPPER)
+            asm volatile("" : "+v"(a_lane_upper[jj]));
+    }
 
     struct BStage
     {
@@ -278,16 +304,20 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
     constexpr int A_RING = 4; // slots; A_AHEAD + 1 are in use
     static_assert(ITERS % A_RING == 0, "a step starts on slot 0");
     u32x8 a_ring[A_RING];
-    auto a_read = [&](auto const* buf, int it) -> u32x8 // row block it % RB, instruction it / RB of a tile row
+    auto a_read = [&](auto buf, int it) -> u32x8 // row block it % RB, instruction it / RB of a tile row
     {
-        char const* const at = reinterpret_cast<char const*>(buf) + (it % RB) * 4096 + (it / RB) * 1024;
-        u32x4 const lo = *reinterpret_cast<u32x4 const*>(at + a_lane_off[0]);
-        u32x4 const hi = *reinterpret_cast<u32x4 const*>(at + a_lane_off[1]);
-        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        typedef __attribute__((address_space(3))) char const lds_char;
+        typedef __attribute__((address_space(3))) u32x4 const lds_u32x4;
+        auto const at = [&](int jj) -> u32x4
+        {
+            uint32_t const c = (uint32_t) ((it % RB) * 4096 + (it / RB) * 1024);
+            return *(lds_u32x4*) ((lds_char*) buf.data + (buf.upper ? a_lane_upper[jj] + (c - kLdsReach) : a_lane_off[jj] + c));
+        };
+        return __builtin_shufflevector(at(0), at(1), 0, 1, 2, 3, 4, 5, 6, 7);
     };
     u32x8 b[KI]; // converted weights, by instruction along K
-    auto compute = [&](auto first_tag, auto const* buf, auto const* buf_after, Fp8Table const& T, Fp8Table& T_next,
-                       BStage const& st, BStage const& st_next, auto* buf_req, int kt_a, TileCtx const& xa, BStage& st_req,
+    auto compute = [&](auto first_tag, auto buf, auto buf_after, Fp8Table const& T, Fp8Table& T_next,
+                       BStage const& st, BStage const& st_next, auto buf_req, int kt_a, TileCtx const& xa, BStage& st_req,
                        int kt_w, TileCtx const& xw) __attribute__((always_inline))
     {
         constexpr bool FIRST = decltype(first_tag)::value;
@@ -365,7 +395,7 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
     BStage st0, st1, st2, st3;
     Fp8Table t0, t1;
     fp8_saturation_on(); // the conversions rely on it; off again before the epilogue
-    auto request_a = [&](auto* buf, int kt)
+    auto request_a = [&](auto buf, int kt)
     {
         uint32_t const base = dma_base(kt, cur);
 #pragma unroll
@@ -405,8 +435,8 @@ __global__ void __launch_bounds__(kW4a8Waves * 64) __attribute__((amdgpu_waves_p
     auto step_barrier = [&]()
     { asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(DEEP ? DMA_OPS + FETCH_OPS : FETCH_OPS) : "memory"); };
     std::false_type const plain{};
-    auto deep_step = [&](auto tag, auto const* buf, auto const* buf_after, Fp8Table const& T, Fp8Table& T_next, BStage const& st,
-                         BStage const& st_next, auto* buf_req, BStage& st_req, int kt, TileCtx const& x) __attribute__((always_inline))
+    auto deep_step = [&](auto tag, auto buf, auto buf_after, Fp8Table const& T, Fp8Table& T_next, BStage const& st,
+                         BStage const& st_next, auto buf_req, BStage& st_req, int kt, TileCtx const& x) __attribute__((always_inline))
     {
         compute(tag, buf, buf_after, T, T_next, st, st_next, buf_req, kt, x, st_req, kt, x);
         step_barrier();

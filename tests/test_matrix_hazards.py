@@ -14,6 +14,7 @@ import subprocess
 import pytest
 
 LLVM_OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+LLVM_READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 WRITE_TO_MATRIX = 2
 # wait states the compiler puts between the builtin and an ordinary reader of its result: 4, 8 and 16 passes
 RESULT = {"16x16x32": 8, "16x16x128": 12, "32x32x16": 12, "32x32x64": 20}
@@ -131,12 +132,31 @@ def _hazards_of(part):
     return found
 
 
-@pytest.mark.skipif(not os.path.exists(LLVM_OBJDUMP), reason="no disassembler")
-def test_built_kernels_keep_the_wait_states(pkg, tmp_path):
-    shutil.copy(pkg.lib_path(), tmp_path / "lib.so")
-    subprocess.run([LLVM_OBJDUMP, "--offloading", "lib.so"], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
-    parts = sorted(tmp_path.glob("*gfx950*"))
+@pytest.fixture(scope="module")
+def device_code(pkg, tmp_path_factory):
+    if not os.path.exists(LLVM_OBJDUMP):
+        pytest.skip("no disassembler")
+    folder = tmp_path_factory.mktemp("code")
+    shutil.copy(pkg.lib_path(), folder / "lib.so")
+    subprocess.run([LLVM_OBJDUMP, "--offloading", "lib.so"], cwd=folder, check=True, stdout=subprocess.DEVNULL)
+    parts = sorted(folder.glob("*gfx950*"))
     assert parts, "no device code in %s" % pkg.lib_path()
+    return parts
+
+
+def test_w4a8_persistent_loops_keep_their_registers(device_code):
+    """No scratch memory in the persistent W4A8 forms: a reload in the loop waits for every request in flight."""
+    seen = {}
+    for part in device_code:
+        notes = subprocess.run([LLVM_READELF, "--notes", str(part)], check=True, stdout=subprocess.PIPE, text=True).stdout
+        for name, scratch in re.findall(r"\.name:\s+(\S+).*?\.private_segment_fixed_size:\s+(\d+)", notes, re.S):
+            if re.match(r"_ZN3woq16gemm_w4a8_kernelILi1ELb[01]ELi16ELb0ELi[12]E", name):
+                seen[name] = int(scratch)
+    assert len(seen) == 4 and not any(seen.values()), seen
+
+
+def test_built_kernels_keep_the_wait_states(pkg, device_code):
+    parts = device_code
     with concurrent.futures.ProcessPoolExecutor(4) as pool:
         found = sum(pool.map(_hazards_of, parts), [])
     assert not found, "%d hazards, the first: %s" % (len(found), found[:8])
