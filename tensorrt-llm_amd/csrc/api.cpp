@@ -1058,7 +1058,8 @@ extern "C" int woq_matmul(const woq_matmul_args* args, void* stream)
 // done before a K split's second launch, nor up to eight rows, where it reads at the memory's rate.
 static bool tiled_w4a8_is_faster(MatmulProblem const& p, GemmPlan& plan)
 {
-    if (!p.w4a8 || !p.built_in_choice || p.m <= 8)
+    // (as for the mid-M kernel: the tiled one moves activations by DMA in 16-byte pieces, the streaming ones load them to registers)
+    if (!p.w4a8 || !p.built_in_choice || p.m <= 8 || reinterpret_cast<uintptr_t>(p.act) % 16)
         return false;
     size_t const asked = plan_gemm_w4a8(p.m, p.n, p.k).ws_bytes, given = p.workspace ? p.workspace_bytes : 0;
     plan = plan_gemm_w4a8(p.m, p.n, p.k, asked < given ? asked : given, false);

@@ -458,6 +458,25 @@ def test_w4a8_tiled_every_tile_count(pkg, oracle, dev, woq_env, rt, with_zeros, 
             assert (out == oracle.round_f16(0.5 * w8[hot])).all(), (tiles, splits)
 
 
+def test_w4a8_few_rows_need_aligned_activations_for_the_tiled_kernel(pkg, oracle, dev):
+    """e4m3 activations that start 8 bytes into an allocation stay on the streaming kernel, with the same result."""
+    F = pkg.functional
+    M, K, N = 16, 14336, 1024
+    prob = oracle.make_w4a8_problem(M, K, N, seed=3, out_dtype="bf16")
+    a8 = oracle.apply_per_channel_scale(prob["act"], prob["pre_quant_scale"], "bf16", "fp8")
+    ref = oracle.woq_matmul_ref(a8, prob["q"], prob["scales"], None, None, None, prob["alpha"], 128, "bf16", w4a8=True)
+    w, sc = preprocess(pkg, oracle, prob["q"], 4, torch.float8_e4m3fn).to(dev), to_dev(prob["scales"], "fp16", dev)
+    room = torch.zeros(M * K + 16, dtype=torch.float8_e4m3fn, device=dev)
+    for skip, tiled in ((16, True), (8, False)):
+        act = room[skip:skip + M * K].view(M, K)
+        act.copy_(torch.from_numpy(a8).to(dev).to(torch.float8_e4m3fn))
+        out = F.woq_matmul_raw(act, None, w, sc, None, None, n=N, k=K, group_size=128, quant_algo=F.FP8_ALPHA,
+                               alpha=prob["alpha"], out_dtype=torch.bfloat16)
+        torch.cuda.synchronize()
+        assert ("gemm w4a8" in _launch(pkg)) == tiled, _launch(pkg)
+        assert oracle.max_rel_err(out.float().cpu().numpy(), ref) < TOL
+
+
 def test_w4a8_few_rows_on_the_tiled_kernel(pkg, oracle, dev):
     """Nine to 32 rows of a long product run on the tiled kernel; its workspace stays the one that the size query
     names, a smaller one is refused as before, and the library's own device array gives the same bits."""
