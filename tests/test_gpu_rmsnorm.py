@@ -73,10 +73,10 @@ def test_rmsnorm_feeds_the_matmul(pkg, oracle, dev):
     assert torch.equal(fused, two_step)
 
 
-@pytest.mark.parametrize("k", [4096, 4104])
+@pytest.mark.parametrize("k", [4104, 8200, 16392])
 def test_rmsnorm_rows_do_not_depend_on_their_number(pkg, oracle, dev, k):
     """Beyond 1024 rows of more than 4096 elements the tables are read behind the sum of squares: the bits of the launch
-    that requests them with the row."""
+    that requests them with the row.  One length for each of the two forms, and one whose end is read again from memory."""
     F = pkg.functional
     x, gamma, b, s = _case(oracle, 1030, k, "bf16", True, True, seed=k)
     xs, rest = to_dev(x, "bf16", dev), [to_dev(gamma, "bf16", dev), to_dev(s, "bf16", dev), 1e-5, to_dev(b, "bf16", dev)]

@@ -477,6 +477,62 @@ def test_w4a8_few_rows_need_aligned_activations_for_the_tiled_kernel(pkg, oracle
         assert oracle.max_rel_err(out.float().cpu().numpy(), ref) < TOL
 
 
+def test_w4a8_nine_rows_and_the_estimates(pkg, dev):
+    """9 ... 14 rows of narrow matrices, by which kernel was measured the faster one by 7 % or more."""
+    F = pkg.functional
+    for K, N, M, tiled in ((14336, 2048, 9, False), (14336, 2048, 10, False), (8192, 1024, 14, False), (14336, 4096, 14, False),
+                           (14336, 1024, 14, True), (28672, 1024, 9, True), (28672, 4096, 12, True)):
+        w = torch.zeros(K // 2 * N, dtype=torch.int8, device=dev)
+        F.woq_matmul_raw(torch.zeros(M, K, dtype=torch.float8_e4m3fn, device=dev), None, w,
+                         torch.ones(K // 128, N, dtype=torch.float16, device=dev), None, None, n=N, k=K, group_size=128,
+                         quant_algo=F.FP8_ALPHA, out_dtype=torch.bfloat16)
+        torch.cuda.synchronize()
+        assert ("gemm w4a8" in _launch(pkg)) == tiled, (K, N, M, _launch(pkg))
+
+
+@pytest.mark.parametrize("K,N,M", [(14336, 1024, 12), (14336, 1024, 16), (8192, 1024, 17), (8192, 1024, 19)])
+@pytest.mark.parametrize("with_zeros", [False, True])
+def test_w4a8_streaming_regime_on_the_tiled_kernel(pkg, oracle, dev, K, N, M, with_zeros):
+    """Problems of the streaming regime whose rows are estimated faster on the tiled kernel: it is the one that runs, with as
+    many K slices as the workspace holds, the same bits in any workspace that holds all and in the library's own
+    array; the streaming kernel runs without room and where the caller names it."""
+    F, lib = pkg.functional, pkg._lib.lib
+    algo = F.FP8_ALPHA | (F.ZERO if with_zeros else 0)
+    assert lib.woq_select_regime(M, N, K, algo) == STREAM
+    prob = oracle.make_w4a8_problem(M, K, N, seed=M, out_dtype="bf16")
+    rng = np.random.default_rng(M)
+    z = oracle.round_f16((rng.standard_normal((K // 128, N)) * 20).astype(np.float32)) if with_zeros else None
+    a8 = oracle.apply_per_channel_scale(prob["act"], prob["pre_quant_scale"], "bf16", "fp8")
+    ref = oracle.woq_matmul_ref(a8, prob["q"], prob["scales"], z, None, None, prob["alpha"], 128, "bf16", w4a8=True)
+    operands = (torch.from_numpy(a8).to(dev).to(torch.float8_e4m3fn), None,
+                preprocess(pkg, oracle, prob["q"], 4, torch.float8_e4m3fn).to(dev), to_dev(prob["scales"], "fp16", dev),
+                None if z is None else to_dev(z, "fp16", dev), None)
+
+    def run(**how):
+        out = F.woq_matmul_raw(*operands, n=N, k=K, group_size=128, quant_algo=algo, alpha=prob["alpha"],
+                               out_dtype=torch.bfloat16, **how)
+        torch.cuda.synchronize()
+        got = out.float().cpu().numpy()
+        assert oracle.max_rel_err(got, ref) < TOL, (_launch(pkg), how)
+        return got, _launch(pkg)
+
+    full, launch = run()
+    assert "gemm w4a8 rt=4 splits=" in launch, launch
+    splits = int(launch.split("splits=")[1].split()[0])
+    need = lib.woq_workspace_bytes(M, N, K, algo, F._WOQ_DT[torch.float8_e4m3fn])
+    slabs = splits * M * N * 4
+    assert splits > 2 and slabs <= need
+    room = torch.full((4 * need,), 0x7F, dtype=torch.uint8, device=dev)
+    for how in (dict(workspace=room[:need]), dict(workspace=room), dict(static_scratch=True)):
+        same, again = run(**how)
+        assert again == launch and (same == full).all(), (again, launch)
+    _, fewer = run(workspace=room[:slabs // 2])  # half the slabs: fewer slices, or the streaming kernel
+    assert "stream" in fewer or int(fewer.split("splits=")[1].split()[0]) <= splits // 2, fewer
+    for how in (dict(workspace=room[:16]), dict(workspace=room[:need], regime=STREAM)):
+        _, other = run(**how)
+        assert "stream" in other, other
+
+
 def test_w4a8_few_rows_on_the_tiled_kernel(pkg, oracle, dev):
     """Nine to 32 rows of a long product run on the tiled kernel; its workspace stays the one that the size query
     names, a smaller one is refused as before, and the library's own device array gives the same bits."""
