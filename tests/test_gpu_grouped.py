@@ -227,3 +227,24 @@ def test_grouped_flexible_group_sizes(pkg, oracle, dev, woq_env, group, K, zero,
         out = run_grouped(pkg, oracle, dev, p, regime=regime)
         assert np.isfinite(out).all()
         assert oracle.max_rel_err(out, ref) < TOL, kernel
+
+
+@pytest.mark.parametrize("rows,K,N,bits,group,want", [
+    (520, 2304, 11264, 4, 128, "skinny rt=4"),            # group scales: stays with the kernel that does not round scaled weights
+    (840, 8576, 3200, 4, 64, "skinny rt=4"),
+    (840, 5632, 2304, 4, 64, "exact rt=4 splits=1 persistent=0 columns=256"),  # one round of 64-row tiles
+    (646, 8576, 3200, 4, 64, "exact rt=4 splits=1 persistent=0 columns=256"),
+    (1200, 2304, 11264, 4, 64, "heights by expert"),
+    (646, 14336, 4096, 4, 0, "skinny rt=4"),              # per-channel: not clearly slower there
+])
+def test_grouped_kernel_choice(pkg, dev, rows, K, N, bits, group, want):
+    F, dt = pkg.functional, torch.bfloat16
+    ends = torch.tensor([rows * (e + 1) // 8 for e in range(8)], dtype=torch.int64, device=dev)
+    w = torch.zeros(8, K * N * bits // 8, dtype=torch.int8, device=dev)
+    scales = torch.ones(*((8, K // group, N) if group else (8, N)), dtype=dt, device=dev)
+    out = F.woq_grouped_matmul_raw(torch.ones(rows, K, dtype=dt, device=dev), w, scales, None, None, ends, n=N, k=K, group_size=group,
+                                   quant_algo=0)
+    torch.cuda.synchronize()
+    launch = pkg._lib.lib.woq_last_launch().decode()
+    assert launch.endswith(want) or want in launch and "exact" not in want, launch
+    assert (out == -8.0 * K).all()
