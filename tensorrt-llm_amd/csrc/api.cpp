@@ -811,16 +811,15 @@ extern "C" void woq_reload_env(void)
 extern "C" int woq_select_regime(int32_t m, int32_t n, int32_t k, int32_t quant_algo)
 {
     // W4A8: the streaming kernel converts every weight to e4m3 in registers and still runs at
-    // memory speed for one 16-row tile; with two tiles per wavefront (17..32 rows) it still beats the
-    // fp8 GEMM kernel, whose 64-row tiles convert the same weights for a quarter of the rows, by 8-39 %
-    // on the Llama-3-8B / 70B shapes - except on the long-K, narrow-N ones from some row count on (below);
-    // beyond that the GEMM kernel
+    // memory speed for one 16-row tile, and with two tiles per wavefront (17..32 rows) it beat the
+    // fp8 GEMM kernel that the regimes were laid down with, except on long-K, narrow-N matrices from some row count on
+    // (below).  They say what a call has to bring, and stay; which kernel runs a problem of this regime from nine
+    // rows on is tiled_w4a8_is_faster's choice
     if (quant_algo & WOQ_ALGO_FP8_ALPHA)
     {
         if (m <= kStreamW4a8AutoMaxM)
             return WOQ_REGIME_STREAM;
-        // (long K on few columns: 28672 x 8192 streams up to 30 rows - 28 rows 52.2 against 57.0 us - 14336 x 4096
-        // up to 19: 24 rows 25.8 against 22.7)
+        // (long K on few columns, against that kernel: 28672 x 8192 up to 30 rows, 14336 x 4096 up to 19)
         if (m <= kStreamW4a8MaxM && !(m > (n <= 4096 ? 19 : 30) && k >= 2 * n))
             return WOQ_REGIME_STREAM;
         return WOQ_REGIME_GEMM;
@@ -1053,9 +1052,11 @@ extern "C" int woq_matmul(const woq_matmul_args* args, void* stream)
 
 // W4A8 problems whose regime is the streaming one may run on the tiled kernel all the same from nine rows on: within the
 // slabs its plan was asked for at that row count, as far as the caller brought them (woq_workspace_bytes covers them).
-// It is taken where it is estimated 7 % cheaper - 28672 x 8192 at 16 / 32 rows 32.7 -> 26.0 / 57.0 -> 27.3 us, 14336 x 4096
-// 16.7 -> 13.8 / 31.3 -> 14.9, 8192 x 57344 at 32 rows 76.9 -> 52.8 - not on small matrices, where the streaming kernel is
-// done before a K split's second launch, nor up to eight rows, where it reads at the memory's rate.
+// It is taken where it is estimated 7 % cheaper - us, streaming -> tiled: 28672 x 8192 at 16 / 17 / 30 rows 32.9 -> 31.8 / 39.2 ->
+// 31.8 / 54.3 -> 33.1, 14336 x 4096 at 16 / 19 rows 16.1 -> 14.4 / 22.6 -> 14.7, 8192 x 57344 at 17 / 32 rows 59.4 -> 56.9 / 77.6
+// -> 56.9, 28672 x 2048 at 9 rows 19.8 -> 15.4 (of 57 such problems measured none is slower) - not on small
+// matrices, where the streaming kernel is done before a K split's second launch, nor up to eight rows, where it reads at
+// the memory's rate.
 static bool tiled_w4a8_is_faster(MatmulProblem const& p, GemmPlan& plan)
 {
     // (as for the mid-M kernel: the tiled one moves activations by DMA in 16-byte pieces, the streaming ones load them to registers)

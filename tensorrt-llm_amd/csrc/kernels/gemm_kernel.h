@@ -704,11 +704,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 
 // few tiles of up to 128 rows as they fit, all of one height, and runs the loop of that height.  All heights share
 // the 128-row loop's registers and LDS: two workgroups a CU.
 // Measured (8 experts, top-2 of T tokens, us, common height -> by expert): 4096 x 28672 with SwiGLU, fp16 per-channel, 150 /
-// 300 / 600 / 1000 tokens 151 -> 122 / 203 -> 162 / 324 -> 283 / 459 -> 384; bf16 group 128 at 300 / 600 tokens 268 -> 193 /
-// 384 -> 330; int8 at 300 288 -> 224.  About half of that is the order of the tiles: with the launch's upper bound of row
+// 300 / 600 / 1000 tokens 151 -> 122 / 203 -> 162 / 324 -> 283 / 459 -> 384; bf16 group 128 at 600 tokens 384 -> 330; int8 at 300
+// 288 -> 224.  About half of that is the order of the tiles: with the launch's upper bound of row
 // tiles dealt to the XCDs, the empty ones at its end left one or two XCDs idle (without that the first came out at 231).
 // What bounds it: conversions and matrix instructions in series (0.735 + 0.117 h us per 128 rows of K and tile of h row
-// tiles, two workgroups a CU), and the tallest expert's tile where the launch is a single round.
+// tiles, two workgroups a CU; 300 tokens: vector unit 67 % of the cycles, matrix core 60 %, both at once 22 %,
+// profiles/grouped_heights_by_expert.md), and the tallest expert's tile where the launch is a single round: 64-row tiles are
+// the faster ones there (plan_grouped).
 template <int DT, int BITS, int GROUP, bool ZERO>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm_flex_kernel(GemmParams p)
 {

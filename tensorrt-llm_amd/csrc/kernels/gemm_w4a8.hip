@@ -25,9 +25,10 @@
 // PFLOP/s), 8192 x 57344 at 128 / 256 rows 119 -> 69.6 / 116 -> 107, 4096 x 4096 at 1990 rows 54.3 -> 36.2 (128-row tiles).
 // With zero-points, on another box: 4096 x 28672 at 1990 / 8192 rows 255 -> 200 / 908 -> 753, 8192 x 57344 at 1024 rows 475 -> 393.
 // By step, 8192 x 57344 at 128 rows: 32x32x64 109, eight wavefronts 88, three steps ahead 75, look-up conversion 70.
-// What bounds it: 128-row tiles the conversions (140 issue slots of each wavefront a step beside 8 instructions of 64
-// cycles); 256-row ones the LDS (every wavefront reads the whole activation tile: 2048 + 256 cycles a step, as many as the
-// matrix core is busy) and, at 8192 rows, the clock.
+// What bounds it (profiles/gemm_w4a8_gate_up_m4096.md): 128-row tiles the conversions (8192 x 57344 at 128 rows: the vector unit
+// issues for 68 % of the cycles, the matrix core is busy for 53 %, and half of the vector work runs under matrix
+// instructions); 256-row ones the matrix core (4096 x 28672 at 4096 rows: busy for 76 %; vector unit 54 %, LDS 38 %) and the clock
+// that it brings down to 1.54 GHz.
 #include "gemm_common.h"
 #include "w4a8_common.h"
 
