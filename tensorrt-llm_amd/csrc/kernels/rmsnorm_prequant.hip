@@ -28,7 +28,8 @@ __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void c
     // trip to memory (us, bf16 -> e4m3 with smoothing: 8 x 8192 3.80 -> 3.46, 1990 x 4096 7.64 -> 6.95, 4096 x 4096 13.6 ->
     // 12.4).  Long rows by the thousand are left as they were: the registers cost residency there (8192 x 8192 42.6 -> 44.4).
     u32x4 const zero = {0u, 0u, 0u, 0u};
-    u32x4 v[CHUNKS], gam[CHUNKS], sca[CHUNKS];
+    u32x4 v[CHUNKS];
+    [[maybe_unused]] u32x4 gam[CHUNKS], sca[CHUNKS];
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i)
     {
@@ -73,8 +74,9 @@ __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void c
     __syncthreads();
     float const inv = __frsqrt_rn((part[0] + part[1] + part[2] + part[3]) / (float) k + eps);
 
-    auto finish = [&](u32x4 w, int piece, u32x4 g, u32x4 sc)
+    auto finish = [&](u32x4 w, int piece, auto const& gamma_piece, auto const& scale_piece) __attribute__((always_inline))
     {
+        u32x4 const g = gamma_piece(piece);
         u32x4 const b = beta ? static_cast<u32x4 const*>(beta)[piece] : u32x4{0u, 0u, 0u, 0u};
         u32x4 y;
 #pragma unroll
@@ -90,6 +92,7 @@ __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void c
         }
         if (scale)
         {
+            u32x4 const sc = scale_piece(piece);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 y[r] = E::mul2(y[r], sc[r]);
@@ -107,21 +110,33 @@ __global__ void __launch_bounds__(256) rmsnorm_prequant_kernel(void* out, void c
         else
             *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(out) + row * k + (long) piece * 8) = y;
     };
+    auto const gamma_read = [&](int piece) { return static_cast<u32x4 const*>(gamma)[piece]; };
+    auto const scale_read = [&](int piece) { return scale ? static_cast<u32x4 const*>(scale)[piece] : zero; };
+    // Not AHEAD: the tables are read where they are used, or both at the top of a piece (us, bf16 -> e4m3 with smoothing: 4096 x 5120
+    // 14.7 and 15.1, 2000 x 5120 7.74 and 7.89; with eight pieces a thread the other way about: 4096 x 14336 36.3 and 34.1, 2000 x 14336
+    // 21.6 and 20.5)
+    constexpr bool TOP = !AHEAD && CHUNKS == 8;
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i)
     {
         int const piece = threadIdx.x + i * 256;
-        if constexpr (!AHEAD)
+        if constexpr (TOP)
         {
-            gam[i] = piece < n8 ? static_cast<u32x4 const*>(gamma)[piece] : zero;
-            sca[i] = piece < n8 && scale ? static_cast<u32x4 const*>(scale)[piece] : zero;
+            gam[i] = piece < n8 ? gamma_read(piece) : zero;
+            sca[i] = piece < n8 ? scale_read(piece) : zero;
         }
-        if (piece < n8)
-            finish(v[i], piece, gam[i], sca[i]);
+        if (piece >= n8)
+            continue;
+        if constexpr (AHEAD || TOP)
+            finish(v[i], piece, [&](int) { return gam[i]; }, [&](int) { return sca[i]; });
+        else
+            finish(v[i], piece, gamma_read, scale_read);
     }
     for (int piece = threadIdx.x + CHUNKS * 256; piece < n8; piece += 256)
-        finish(*reinterpret_cast<u32x4 const*>(src + (long) piece * 8), piece, static_cast<u32x4 const*>(gamma)[piece],
-            scale ? static_cast<u32x4 const*>(scale)[piece] : zero);
+    {
+        u32x4 const g = gamma_read(piece), sc = scale_read(piece);
+        finish(*reinterpret_cast<u32x4 const*>(src + (long) piece * 8), piece, [&](int) { return g; }, [&](int) { return sc; });
+    }
 }
 
 template <int DT, bool TO_FP8>
